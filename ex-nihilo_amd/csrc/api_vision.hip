@@ -76,10 +76,43 @@ float half_to_float(uint16_t h) {
 
 }  // namespace
 
+// what a split product needs of a weight: the largest |x|, the largest row's 2-norm (a vector is
+// one row) and, of a matrix whose values are fp16 times 2^-kw, those fp16 rows (kp apart)
+struct VisFacts {
+  double mx = 0, norm = 0;
+  uint16_t* h = nullptr;
+  int kp = 0, kw = 0;
+  bool exact = false;
+};
+
+// one product of the tower: its fp32 weights and, where SPLIT, the fp16 rows and the exponents of
+// its input's scale (2^ex) and of the weights'
+struct VisMm {
+  const float *w = nullptr, *b = nullptr;
+  const uint16_t* h = nullptr;
+  int n = 0, k = 0, kp = 0, kw = 0, ex = 0;
+  bool split = false;
+  float descale() const { return std::ldexp(1.f, -(ex + kw)); }
+};
+struct VisBlock {
+  const float *ln1w, *ln1b, *ln2w, *ln2b;
+  VisMm qkv, out, up, down;
+  int eq = 0, ek = 0, ev = 0;   // the exponents of split q, k, v
+  bool heads = false;           // attention on split heads
+};
+struct VisMerger {
+  const float *lnw, *lnb;
+  VisMm fc1, fc2;
+};
+
 struct exn_vision {
   exn_ctx* ctx = nullptr;
   std::vector<VExpect> expect;
   std::map<std::string, float*> t;   // fp32 device copies
+  std::map<std::string, VisFacts> facts;
+  std::vector<VisBlock> blocks;       // made from the weights when one changed
+  VisMerger mergers[4];               // deepstack 0 .. 2, then the merger
+  bool plan_ok = false;
   std::map<std::string, Buf> bufs;
   float* pw = nullptr;                // the two patch kernels summed
   bool pw_ok = false;
@@ -119,7 +152,144 @@ static int vis_store(exn_vision* v, const std::string& name, int64_t n, const fl
   if (!p) TRY(dev_alloc((void**)&p, (size_t)n * 4));
   HIPCHK(hipMemcpyAsync(p, data, (size_t)n * 4, hipMemcpyDeviceToDevice, v->ctx->stream));
   if (name.rfind("v.patch_embd.weight", 0) == 0) v->pw_ok = false;
+  v->plan_ok = false;
   return EXN_OK;
+}
+
+// the facts of the stored tensors WHICH (indices of expect): two passes over each on the device,
+// the second, where the values fit, the fp16 rows.  Ends with the stream idle.
+static int vis_measure(exn_vision* v, const std::vector<size_t>& which) {
+  hipStream_t s = v->ctx->stream;
+  float* recp = nullptr;
+  TRY(vis_buf(v, "facts", v->expect.size() * 16, &recp));
+  uint32_t* rec = (uint32_t*)recp;
+  std::vector<uint32_t> host(which.size() * 4);
+  auto dims = [&](size_t i, int64_t& rows, int64_t& cols) {
+    const std::vector<int64_t>& d = v->expect[i].shape;
+    rows = d.size() > 1 ? d[0] : 1;
+    cols = 1;
+    for (size_t k = d.size() > 1 ? 1 : 0; k < d.size(); ++k) cols *= d[k];
+  };
+  // the patch kernels (their input has no bound) and the position table stay fp32
+  auto used = [&](size_t i) { return v->expect[i].name.compare(0, 7, "v.patch") && v->expect[i].name.compare(0, 7, "v.posit"); };
+  auto fetch = [&]() -> int {
+    HIPCHK(hipMemcpyAsync(host.data(), rec, host.size() * 4, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    return EXN_OK;
+  };
+  int64_t rows, cols;
+  HIPCHK(tensor_stats_clear(s, rec, (int64_t)which.size()));
+  for (size_t j = 0; j < which.size(); ++j)
+    if (used(which[j])) {
+      dims(which[j], rows, cols);
+      HIPCHK(vis_stats(s, rows, cols, v->t[v->expect[which[j]].name], rec + 4 * j));
+    }
+  TRY(fetch());
+  for (size_t j = 0; j < which.size(); ++j) {
+    if (!used(which[j])) continue;
+    const VExpect& e = v->expect[which[j]];
+    VisFacts& f = v->facts[e.name];
+    float mx, ss;
+    memcpy(&mx, &host[4 * j], 4);
+    memcpy(&ss, &host[4 * j + 1], 4);
+    f.mx = mx;
+    f.norm = std::sqrt((double)ss) * 1.001;   // the sum's own rounding
+    f.exact = false;
+    if (e.shape.size() < 2 || !std::isfinite(mx)) continue;
+    dims(which[j], rows, cols);
+    f.kp = (int)((cols + 63) / 64 * 64);
+    f.kw = mx > 0.f ? std::min(40, std::max(0, 14 - std::ilogb(mx))) : 0;
+    if (!f.h && dev_alloc((void**)&f.h, (size_t)rows * f.kp * 2) != EXN_OK) continue;   // the fp32 product then
+    f.exact = true;
+    HIPCHK(vis_pack(s, rows, (int)cols, f.kp, std::ldexp(1.f, f.kw), v->t[e.name], f.h, rec + 4 * j + 2));
+  }
+  TRY(fetch());
+  for (size_t j = 0; j < which.size(); ++j)
+    if (used(which[j]) && host[4 * j + 2]) v->facts[v->expect[which[j]].name].exact = false;
+  return EXN_OK;
+}
+
+// the exponent that scales values of at most BOUND to at most 2^15; false where there is none
+static bool vis_exponent(double bound, int& e) {
+  if (!(bound >= 0.0) || !std::isfinite(bound)) return false;
+  e = bound > 0.0 ? std::min(60, 14 - std::ilogb(bound * 1.01)) : 0;
+  return e >= -60;
+}
+
+// The products of the tower and, from the weights alone, which of them run split and at which
+// scales.  LayerNorm's output is at most sqrt(D) max|g| + max|b| (no centred row has an element
+// above sqrt(D) of its deviation), its row norm at most sqrt(D) max|g| + |b|; a product's output
+// at most that norm times the largest weight row's plus max|bias|; the rotary at most sqrt(2)
+// times its input; attention's output and GELU's at most their input.
+static void vis_plan(exn_vision* v) {
+  auto facts = [&](const std::string& n) -> const VisFacts& { return v->facts[n]; };
+  auto mm = [&](const std::string& name) {
+    VisMm r;
+    const VExpect* e = vis_find(v, (name + ".weight").c_str());
+    r.n = (int)e->shape[0];
+    r.k = (int)e->shape[1];
+    r.w = vis_t(v, name + ".weight");
+    r.b = vis_t(v, name + ".bias");
+    const VisFacts& f = facts(name + ".weight");
+    r.h = f.h;
+    r.kp = f.kp;
+    r.kw = f.kw;
+    r.split = f.exact;
+    return r;
+  };
+  // LN's bounds on an element and on a row's norm, from its tensors and its width
+  struct Bound { double el, norm; };
+  auto ln = [&](const std::string& name, int width) {
+    const VisFacts &g = facts(name + ".weight"), &b = facts(name + ".bias");
+    const double r = std::sqrt((double)width) * g.mx;
+    return Bound{r + b.mx, r + b.norm};
+  };
+  auto out = [&](const std::string& name, double norm) { return norm * facts(name + ".weight").norm + facts(name + ".bias").mx; };
+  auto merger = [&](const std::string& norm, const std::string& fc1, const std::string& fc2, int width) {
+    VisMerger m;
+    m.lnw = vis_t(v, norm + ".weight");
+    m.lnb = vis_t(v, norm + ".bias");
+    m.fc1 = mm(fc1);
+    m.fc2 = mm(fc2);
+    const Bound z = ln(norm, width);
+    const double rn = z.norm * std::sqrt(m.fc1.k / (double)width);   // the row is k / width normed ones
+    const bool ok = m.fc1.split && m.fc2.split && vis_exponent(z.el, m.fc1.ex) && vis_exponent(out(fc1, rn), m.fc2.ex);
+    m.fc1.split = m.fc2.split = ok;
+    return m;
+  };
+  v->blocks.clear();
+  char p[64];
+  for (int i = 0; i < kVisDepth; ++i) {
+    snprintf(p, sizeof p, "v.blk.%d.", i);
+    const std::string b = p;
+    VisBlock k;
+    k.ln1w = vis_t(v, b + "ln1.weight");
+    k.ln1b = vis_t(v, b + "ln1.bias");
+    k.ln2w = vis_t(v, b + "ln2.weight");
+    k.ln2b = vis_t(v, b + "ln2.bias");
+    k.qkv = mm(b + "attn_qkv");
+    k.out = mm(b + "attn_out");
+    k.up = mm(b + "ffn_up");
+    k.down = mm(b + "ffn_down");
+    const Bound z1 = ln(b + "ln1", kVisD), z2 = ln(b + "ln2", kVisD);
+    const double head = out(b + "attn_qkv", z1.norm);
+    k.qkv.split = k.qkv.split && vis_exponent(z1.el, k.qkv.ex);
+    k.heads = vis_exponent(head * 1.4143 * 1.4427 / std::sqrt((double)kVisHd), k.eq) &&
+              vis_exponent(head * 1.4143, k.ek) && vis_exponent(head, k.ev);
+    k.out.ex = k.ev;
+    k.out.split = k.out.split && k.heads;
+    const bool ok = k.up.split && k.down.split && vis_exponent(z2.el, k.up.ex) &&
+                    vis_exponent(out(b + "ffn_up", z2.norm), k.down.ex);
+    k.up.split = k.down.split = ok;
+    v->blocks.push_back(k);
+  }
+  for (int j = 0; j < 3; ++j) {
+    snprintf(p, sizeof p, "v.deepstack.%d", kVisDeep[j]);
+    const std::string b = p;
+    v->mergers[j] = merger(b + ".norm", b + ".fc1", b + ".fc2", 4 * kVisD);
+  }
+  v->mergers[3] = merger("v.post_ln", "mm.0", "mm.2", kVisD);
+  v->plan_ok = true;
 }
 
 
@@ -147,6 +317,7 @@ int exn_vision_destroy(exn_vision* v) {
   if (!v) return EXN_OK;
   TRY(exn_vision_release(v));
   for (auto& kv : v->t) dev_free(kv.second);
+  for (auto& kv : v->facts) dev_free(kv.second.h);
   dev_free(v->pw);
   delete v;
   return EXN_OK;
@@ -197,8 +368,7 @@ int exn_vision_set(exn_vision* v, const char* name, int kind, const void* data, 
   HIPCHK(hipMemcpyAsync(tmp, f.data(), (size_t)n * 4, hipMemcpyHostToDevice, v->ctx->stream));
   TRY(vis_store(v, e->name, n, tmp));
   if (table) v->side = side;
-  HIPCHK(hipStreamSynchronize(v->ctx->stream));
-  return EXN_OK;
+  return vis_measure(v, {(size_t)(e - v->expect.data())});
 }
 
 // every tower tensor from the counter generator (the oracle's SynthVision): value = base +
@@ -242,8 +412,9 @@ int exn_vision_synth(exn_vision* v, uint64_t seed) {
     TRY(vis_store(v, nm, n, tmp));
     if (nm == "v.position_embd.weight") v->side = kVisSide;
   }
-  HIPCHK(hipStreamSynchronize(v->ctx->stream));
-  return EXN_OK;
+  std::vector<size_t> all(v->expect.size());
+  for (size_t i = 0; i < all.size(); ++i) all[i] = i;
+  return vis_measure(v, all);
 }
 
 int exn_vision_check(exn_vision* v) {
@@ -262,6 +433,8 @@ int exn_vision_memory(exn_vision* v, int64_t* weights, int64_t* scratch_bytes) {
     for (auto d : e.shape) n *= d;
     if (e.name == "v.position_embd.weight") n = (int64_t)v->side * v->side * kVisD;
     w += n * 4;
+    auto f = v->facts.find(e.name);
+    if (f != v->facts.end() && f->second.h) w += e.shape[0] * f->second.kp * 2;
   }
   if (v->pw) w += (int64_t)kVisD * 768 * 4;
   for (auto& kv : v->bufs) s += (int64_t)kv.second.bytes;
@@ -277,50 +450,86 @@ int exn_vision_trace(exn_vision* v, int on) {
 }
 
 
-// a merger (src/cuda-vision.lisp:71-82; inspect/ref_vision.py:109-118): four patches' rows as
-// one row of 4608, LayerNorm after (deepstack, PREFIX) or before (v.post_ln), fc1, GELU (erf),
-// fc2 into OUT (M x 4096)
-static int vis_merger(exn_vision* v, const float* x, int n, float* out, const char* prefix) {
+// LayerNorm rows (N of WIDTH) of X, first X += BIAS + S parts where a split product left them,
+// into OUT as the product NEXT reads it: split rows or fp32
+static int vis_norm(exn_vision* v, int64_t n, int width, float* x, int S, const float* part, const float* bias,
+                    const float* w, const float* b, const VisMm& next, float* out) {
+  HIPCHK(vis_ln_s(v->ctx->stream, n, width, width, x, S, part, bias, w, b, std::ldexp(1.f, next.ex),
+                  next.split ? (uint16_t*)out : nullptr, next.split ? nullptr : out));
+  return EXN_OK;
+}
+
+// X (M rows, as vis_norm or the product before left them) through MM into fp32 Y, + R
+static int vis_mm(exn_vision* v, const VisMm& mm, const float* x, const float* r, float* y, int64_t m) {
   hipStream_t s = v->ctx->stream;
+  if (mm.split)
+    HIPCHK(vis_gemm_s(s, (const uint16_t*)x, mm.h, mm.b, r, y, nullptr, m, mm.n, mm.kp, mm.descale(), 0.f, 0, 0));
+  else
+    HIPCHK(vis_gemm(s, x, mm.w, mm.b, r, y, m, mm.n, mm.k, 0));
+  return EXN_OK;
+}
+
+// ... and GELU (ACT), as the product NEXT reads it
+static int vis_mm_gelu(exn_vision* v, const VisMm& mm, const VisMm& next, const float* x, float* y, int64_t m, int act) {
+  hipStream_t s = v->ctx->stream;
+  if (mm.split)
+    HIPCHK(vis_gemm_s(s, (const uint16_t*)x, mm.h, mm.b, nullptr, nullptr, (uint16_t*)y, m, mm.n, mm.kp, mm.descale(),
+                      std::ldexp(1.f, next.ex), next.kp, act));
+  else
+    HIPCHK(vis_gemm(s, x, mm.w, mm.b, nullptr, y, m, mm.n, mm.k, act));
+  return EXN_OK;
+}
+
+// X += X's product MM: whole, or its S parts left in PART for the next vis_norm
+static int vis_mm_add(exn_vision* v, const VisMm& mm, const float* in, float* x, int64_t m, int& S, float* part) {
+  S = mm.split ? vis_split(m, mm.n, mm.kp) : 1;
+  if (S > 1) {
+    HIPCHK(vis_gemm_part(v->ctx->stream, (const uint16_t*)in, mm.h, part, m, mm.n, mm.kp, mm.descale(), S));
+    return EXN_OK;
+  }
+  S = 0;
+  return vis_mm(v, mm, in, x, x, m);
+}
+
+// a merger (src/cuda-vision.lisp:71-82; inspect/ref_vision.py:109-118): four patches' rows as
+// one row of 4608, LayerNorm after (deepstack) or before (v.post_ln, MG 3; S, PART and BIAS as
+// vis_norm), fc1, GELU (erf), fc2 into OUT (M x 4096)
+static int vis_merger(exn_vision* v, float* x, int n, int S, const float* part, const float* bias, float* out, int mg) {
   const int m = n / 4, d4 = 4 * kVisD;
+  const VisMerger& g = v->mergers[mg];
   float *t1, *t2;
   TRY(vis_buf(v, "mt1", (size_t)n * kVisD * 4, &t1));
   TRY(vis_buf(v, "mt2", (size_t)m * d4 * 4, &t2));
-  std::string fc1 = "mm.0", fc2 = "mm.2";
-  if (prefix) {
-    const std::string p = prefix;
-    HIPCHK(vis_ln(s, m, d4, x, vis_t(v, p + ".norm.weight"), vis_t(v, p + ".norm.bias"), t1));
-    fc1 = p + ".fc1";
-    fc2 = p + ".fc2";
-  } else {
-    HIPCHK(vis_ln(s, n, kVisD, x, vis_t(v, "v.post_ln.weight"), vis_t(v, "v.post_ln.bias"), t1));
-  }
-  HIPCHK(vis_gemm(s, t1, vis_t(v, fc1 + ".weight"), vis_t(v, fc1 + ".bias"), nullptr, t2, m, d4, d4, 2));
-  HIPCHK(vis_gemm(s, t2, vis_t(v, fc2 + ".weight"), vis_t(v, fc2 + ".bias"), nullptr, out, m, kVisOut, d4, 0));
-  return EXN_OK;
+  if (mg < 3) TRY(vis_norm(v, m, d4, x, S, part, bias, g.lnw, g.lnb, g.fc1, t1));
+  else TRY(vis_norm(v, n, kVisD, x, S, part, bias, g.lnw, g.lnb, g.fc1, t1));
+  TRY(vis_mm_gelu(v, g.fc1, g.fc2, t1, t2, m, 2));
+  return vis_mm(v, g.fc2, t2, nullptr, out, m);
 }
 
 // vision-encode on the device (src/cuda-vision.lisp:34-101)
 static int vis_encode(exn_vision* v, const float* px, int h, int w, float* merged, float* deep) {
   hipStream_t s = v->ctx->stream;
-  const int gh = h / 16, gw = w / 16, n = gh * gw, m = n / 4, D = kVisD;
+  const int gh = h / 16, gw = w / 16, n = gh * gw, m = n / 4, D = kVisD, np = (n + 63) / 64 * 64;
   if (!v->pw_ok) {
     if (!v->pw) TRY(dev_alloc((void**)&v->pw, (size_t)D * 768 * 4));
     HIPCHK(vis_sum(s, (int64_t)D * 768, vis_t(v, "v.patch_embd.weight"), vis_t(v, "v.patch_embd.weight.1"), v->pw));
     v->pw_ok = true;
   }
-  float *pat, *pe, *cs, *x, *hb, *qkv, *q, *k, *vt, *att, *up;
+  if (!v->plan_ok) vis_plan(v);
+  float *pat, *pe, *cs, *x, *hb, *qkv, *q, *k, *vt, *att, *up, *part = nullptr;
   TRY(vis_buf(v, "pat", (size_t)n * 768 * 4, &pat));
   TRY(vis_buf(v, "pe", (size_t)n * D * 4, &pe));
   TRY(vis_buf(v, "cs", (size_t)n * 144 * 4, &cs));
   TRY(vis_buf(v, "x", (size_t)n * D * 4, &x));
   TRY(vis_buf(v, "hb", (size_t)n * D * 4, &hb));
   TRY(vis_buf(v, "qkv", (size_t)n * 3 * D * 4, &qkv));
-  TRY(vis_buf(v, "q", (size_t)n * D * 4, &q));
-  TRY(vis_buf(v, "k", (size_t)n * D * 4, &k));
-  TRY(vis_buf(v, "vt", (size_t)n * D * 4, &vt));
+  TRY(vis_buf(v, "q", (size_t)n * kVisHeads * 304, &q));   // split rows of 304 bytes a head, or fp32 ones of 288
+  TRY(vis_buf(v, "k", (size_t)n * kVisHeads * 304, &k));
+  TRY(vis_buf(v, "vt", (size_t)np * D * 4, &vt));
   TRY(vis_buf(v, "att", (size_t)n * D * 4, &att));
-  TRY(vis_buf(v, "up", (size_t)n * kVisF * 4, &up));
+  TRY(vis_buf(v, "up", (size_t)n * ((kVisF + 63) / 64 * 64) * 4, &up));
+  const int most = std::max(vis_split(n, D, D), vis_split(n, D, (kVisF + 63) / 64 * 64));
+  if (most > 1) TRY(vis_buf(v, "part", (size_t)most * n * D * 4, &part));
   HIPCHK(vis_prep(s, px, w, gh, gw, vis_t(v, "v.position_embd.weight"), v->side, D, pat, pe, cs));
   HIPCHK(vis_gemm(s, pat, v->pw, vis_t(v, "v.patch_embd.bias"), pe, x, n, D, 768, 0));
   float* tr = nullptr;
@@ -329,26 +538,38 @@ static int vis_encode(exn_vision* v, const float* px, int h, int w, float* merge
     HIPCHK(hipMemcpyAsync(tr, x, (size_t)n * D * 4, hipMemcpyDeviceToDevice, s));
   }
   const float qscale = (float)(1.4426950408889634 / sqrt((double)kVisHd));
-  char p[64];
-  for (int i = 0; i < kVisDepth; ++i) {
-    snprintf(p, sizeof p, "v.blk.%d.", i);
-    const std::string b = p;
-    HIPCHK(vis_ln(s, n, D, x, vis_t(v, b + "ln1.weight"), vis_t(v, b + "ln1.bias"), hb));
-    HIPCHK(vis_gemm(s, hb, vis_t(v, b + "attn_qkv.weight"), vis_t(v, b + "attn_qkv.bias"), nullptr, qkv, n, 3 * D, D, 0));
-    HIPCHK(vis_heads(s, n, kVisHeads, qkv, cs, qscale, q, k, vt));
-    HIPCHK(vis_attend(s, n, kVisHeads, q, k, vt, att));
-    HIPCHK(vis_gemm(s, att, vis_t(v, b + "attn_out.weight"), vis_t(v, b + "attn_out.bias"), x, x, n, D, D, 0));
-    HIPCHK(vis_ln(s, n, D, x, vis_t(v, b + "ln2.weight"), vis_t(v, b + "ln2.bias"), hb));
-    HIPCHK(vis_gemm(s, hb, vis_t(v, b + "ffn_up.weight"), vis_t(v, b + "ffn_up.bias"), nullptr, up, n, kVisF, D, 1));
-    HIPCHK(vis_gemm(s, up, vis_t(v, b + "ffn_down.weight"), vis_t(v, b + "ffn_down.bias"), x, x, n, D, kVisF, 0));
-    if (i == 0 && tr) HIPCHK(hipMemcpyAsync(tr + (size_t)n * D, x, (size_t)n * D * 4, hipMemcpyDeviceToDevice, s));
+  int S = 0;                       // the parts that the residual stream still lacks
+  const float* bias = nullptr;     // and their bias
+  for (int i = 0; i <= kVisDepth; ++i) {
+    // block i's first LayerNorm finishes block i - 1's rows, which the merger after i - 1 reads
+    if (i < kVisDepth) {
+      const VisBlock& b = v->blocks[i];
+      TRY(vis_norm(v, n, D, x, S, part, bias, b.ln1w, b.ln1b, b.qkv, hb));
+      S = 0;
+    }
+    if (i == 1 && tr) HIPCHK(hipMemcpyAsync(tr + (size_t)n * D, x, (size_t)n * D * 4, hipMemcpyDeviceToDevice, s));
     for (int j = 0; j < 3; ++j)
-      if (kVisDeep[j] == i) {
-        snprintf(p, sizeof p, "v.deepstack.%d", i);
-        TRY(vis_merger(v, x, n, deep + (size_t)j * m * kVisOut, p));
-      }
+      if (kVisDeep[j] == i - 1) TRY(vis_merger(v, x, n, 0, nullptr, nullptr, deep + (size_t)j * m * kVisOut, j));
+    if (i == kVisDepth) break;
+    const VisBlock& b = v->blocks[i];
+    TRY(vis_mm(v, b.qkv, hb, nullptr, qkv, n));
+    if (b.heads) {
+      HIPCHK(vis_heads_s(s, n, np, kVisHeads, qkv, cs, std::ldexp(qscale, b.eq), std::ldexp(1.f, b.ek),
+                         std::ldexp(1.f, b.ev), (uint16_t*)q, (uint16_t*)k, (uint16_t*)vt));
+      HIPCHK(vis_attend_s(s, n, np, kVisHeads, (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)vt,
+                          std::ldexp(1.f, -(b.eq + b.ek)), std::ldexp(1.f, -b.ev), D, b.out.split ? (uint16_t*)att : nullptr,
+                          b.out.split ? nullptr : att));
+    } else {
+      HIPCHK(vis_heads(s, n, kVisHeads, qkv, cs, qscale, q, k, vt));
+      HIPCHK(vis_attend(s, n, kVisHeads, q, k, vt, att));
+    }
+    TRY(vis_mm_add(v, b.out, att, x, n, S, part));
+    TRY(vis_norm(v, n, D, x, S, part, b.out.b, b.ln2w, b.ln2b, b.up, hb));
+    TRY(vis_mm_gelu(v, b.up, b.down, hb, up, n, 1));
+    TRY(vis_mm_add(v, b.down, up, x, n, S, part));
+    bias = b.down.b;
   }
-  TRY(vis_merger(v, x, n, merged, nullptr));
+  TRY(vis_merger(v, x, n, S, part, bias, merged, 3));
   if (tr) v->traced_n = n;
   return EXN_OK;
 }

@@ -325,6 +325,27 @@ hipError_t vis_heads(hipStream_t s, int n, int heads, const float* qkv, const fl
 hipError_t vis_attend(hipStream_t s, int n, int heads, const float* q, const float* k, const float* vt, float* att);
 hipError_t vis_sum(hipStream_t s, int64_t n, const float* a, const float* b, float* y);
 hipError_t round_f16(hipStream_t s, int64_t n, float* x);
+// ... and on fp16 parts of fp32 values (vision_split.hip): a split row is 2 KP halves, 32 hi then
+// 32 lo for every 32 columns.  vis_stats: the bits of max |x| and of the largest row's sum of
+// squares into rec[0], rec[1] (cleared first).  vis_pack: SCALE x as fp16 rows of KP, *INEXACT
+// set where a value changes.  vis_ln_s: X += BIAS + S parts (rows x width floats each), then
+// LayerNorm into YS (times SCALE) or fp32 YF.  vis_gemm_s: DESCALE X W^T + bias (+ R) into Y, or
+// through GELU, times OSCALE, into split rows YS of LDY; vis_gemm_part: its S parts over K
+// (vis_split: how many pay).  vis_heads_s, vis_attend_s: heads and attention
+hipError_t vis_stats(hipStream_t s, int64_t rows, int64_t cols, const float* x, uint32_t* rec);
+hipError_t vis_pack(hipStream_t s, int64_t rows, int K, int KP, float scale, const float* x, uint16_t* y,
+                    uint32_t* inexact);
+hipError_t vis_ln_s(hipStream_t s, int64_t rows, int width, int kp, float* x, int S, const float* part,
+                    const float* bias, const float* w, const float* b, float scale, uint16_t* ys, float* yf);
+hipError_t vis_gemm_s(hipStream_t s, const uint16_t* x, const uint16_t* w, const float* bias, const float* r, float* y,
+                      uint16_t* ys, int64_t M, int64_t N, int64_t KP, float descale, float oscale, int64_t ldy, int act);
+int vis_split(int64_t M, int64_t N, int64_t KP);
+hipError_t vis_gemm_part(hipStream_t s, const uint16_t* x, const uint16_t* w, float* part, int64_t M, int64_t N,
+                         int64_t KP, float descale, int S);
+hipError_t vis_heads_s(hipStream_t s, int n, int np, int heads, const float* qkv, const float* cs, float qs, float ks,
+                       float vs, uint16_t* q, uint16_t* k, uint16_t* vt);
+hipError_t vis_attend_s(hipStream_t s, int n, int np, int heads, const uint16_t* q, const uint16_t* k, const uint16_t* vt,
+                        float sc, float vde, int kp, uint16_t* ys, float* yf);
 
 // the prompt encoder (encoder.hip): the token embedding's rows, Q8_0 (qs, d) or fp32 (f32)
 hipError_t enc_embed(hipStream_t s, const int32_t* ids, int n, int64_t vocab, const int8_t* qs, const uint16_t* d,

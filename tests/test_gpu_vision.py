@@ -189,6 +189,41 @@ def test_encode_reads_a_table_of_another_side_and_f16_tensors(ctx, owt):
         v.destroy()
 
 
+@pytest.mark.parametrize("hw", [(32, 32), (32, 544), (96, 352)])
+def test_encode_with_split_and_fp32_products(ctx, owt, hw):
+    """Products on fp16 parts and in fp32 side by side, at 4, 68 and 132 patches (one past a tile of
+    64 rows and of 128): block 0's QKV and block 1's down matrices and a merger's fc1 hold values
+    that fp16 cannot (their products stay fp32, the neighbours' rows change format); block 2's
+    up matrix is 2^-12 of its LayerNorm's gain times 2^12, so its scales move and nothing else.
+    The bar is the whole tower's: float32 arithmetic in another order over 27 blocks."""
+    wt = vo.SynthVision(SEED, vo.VShape())
+    wt.cache = dict(owt.cache)
+    v = X.Vision(ctx)
+    try:
+        for name, shape in vo.vision_expected(vo.VShape()):
+            a = wt(name)
+            if name in ("v.blk.0.attn_qkv.weight", "v.blk.1.ffn_down.weight", "v.deepstack.8.fc1.weight"):
+                a = (a * np.float32(1.0 + 2.0 ** -14)).astype(np.float32)
+            elif name.startswith("v.blk.2.ln2."):
+                a = a * np.float32(4096.0)
+            elif name == "v.blk.2.ffn_up.weight":
+                a = a * np.float32(2.0 ** -12)
+            wt.cache[name] = a
+            v.set(name, X.F32, a, shape)
+        h, w = hw
+        px = vo.synth_picture(SEED + 8, h, w)
+        v.trace(True)
+        merged, deep, m = X.vision_encode(v, px, h, w)
+        blk0 = v.traced(1, 4 * m)
+        want = vo.encode(px, wt)
+        errs = [xo.rel_l2(blk0, want["blk0"]), xo.rel_l2(merged, want["merged"])] + \
+               [xo.rel_l2(deep[j], want["ds"][j]) for j in range(3)]
+        say("split and fp32", hw, errs)
+        assert errs[0] < 1e-5 and max(errs) < 1e-4
+    finally:
+        v.destroy()
+
+
 def test_release_frees_scratch_and_keeps_weights(tower):
     """vision-release (src/cuda-vision.lisp:103-107): the scratch freed, the weights kept; the
     next encode makes its buffers again and gives the same rows bit for bit."""
