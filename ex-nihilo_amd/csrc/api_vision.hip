@@ -54,26 +54,6 @@ std::vector<VExpect> vision_expected() {
   return r;
 }
 
-// fp16 bits -> fp32, subnormals, infinities and NaNs kept
-float half_to_float(uint16_t h) {
-  const uint32_t sign = (uint32_t)(h & 0x8000u) << 16, e = (h >> 10) & 0x1Fu, m = h & 0x3FFu;
-  uint32_t u;
-  if (e == 0x1F) {
-    u = sign | 0x7F800000u | (m << 13);
-  } else if (e != 0) {
-    u = sign | ((e + 112) << 23) | (m << 13);
-  } else if (m == 0) {
-    u = sign;
-  } else {
-    float f = (float)m * 5.9604644775390625e-08f;   // m * 2^-24, exact
-    memcpy(&u, &f, 4);
-    u |= sign;
-  }
-  float f;
-  memcpy(&f, &u, 4);
-  return f;
-}
-
 }  // namespace
 
 // what a split product needs of a weight: the largest |x|, the largest row's 2-norm (a vector is
@@ -199,7 +179,7 @@ static int vis_measure(exn_vision* v, const std::vector<size_t>& which) {
     dims(which[j], rows, cols);
     f.kp = (int)((cols + 63) / 64 * 64);
     f.kw = mx > 0.f ? std::min(40, std::max(0, 14 - std::ilogb(mx))) : 0;
-    if (!f.h && dev_alloc((void**)&f.h, (size_t)rows * f.kp * 2) != EXN_OK) continue;   // the fp32 product then
+    if (!f.h && dev_alloc((void**)&f.h, (size_t)((rows + 63) / 64 * 64) * f.kp * 2) != EXN_OK) continue;   // the fp32 product then
     f.exact = true;
     HIPCHK(vis_pack(s, rows, (int)cols, f.kp, std::ldexp(1.f, f.kw), v->t[e.name], f.h, rec + 4 * j + 2));
   }
@@ -345,27 +325,20 @@ int exn_vision_set(exn_vision* v, const char* name, int kind, const void* data, 
   }
   int64_t n = 1;
   for (int i = 0; i < ndims; ++i) n *= dims[i];
-  std::vector<float> f((size_t)n);
-  if (kind == EXN_F32) {
-    memcpy(f.data(), data, (size_t)n * 4);
-  } else if (kind == EXN_F16) {
-    const uint16_t* h = (const uint16_t*)data;
-    for (int64_t i = 0; i < n; ++i) f[(size_t)i] = half_to_float(h[i]);
-  } else {
-    const uint16_t* b = (const uint16_t*)data;
-    for (int64_t i = 0; i < n; ++i) {
-      const uint32_t u = (uint32_t)b[i] << 16;
-      memcpy(&f[(size_t)i], &u, 4);
-    }
-  }
   if (table && v->t.count(e->name) && v->side != side) {
     HIPCHK(hipStreamSynchronize(v->ctx->stream));
     dev_free(v->t[e->name]);
     v->t.erase(e->name);
   }
   float* tmp = nullptr;
-  TRY(ctx_tmp(v->ctx, (size_t)n * 4, (void**)&tmp));
-  HIPCHK(hipMemcpyAsync(tmp, f.data(), (size_t)n * 4, hipMemcpyHostToDevice, v->ctx->stream));
+  TRY(ctx_tmp(v->ctx, (size_t)n * 6, (void**)&tmp));   // fp32 values, and behind them the 16-bit ones as given
+  if (kind == EXN_F32) {
+    HIPCHK(hipMemcpyAsync(tmp, data, (size_t)n * 4, hipMemcpyHostToDevice, v->ctx->stream));
+  } else {
+    uint16_t* raw = (uint16_t*)(tmp + n);
+    HIPCHK(hipMemcpyAsync(raw, data, (size_t)n * 2, hipMemcpyHostToDevice, v->ctx->stream));
+    HIPCHK(vis_widen(v->ctx->stream, n, raw, kind == EXN_BF16, tmp));
+  }
   TRY(vis_store(v, e->name, n, tmp));
   if (table) v->side = side;
   return vis_measure(v, {(size_t)(e - v->expect.data())});
@@ -434,7 +407,7 @@ int exn_vision_memory(exn_vision* v, int64_t* weights, int64_t* scratch_bytes) {
     if (e.name == "v.position_embd.weight") n = (int64_t)v->side * v->side * kVisD;
     w += n * 4;
     auto f = v->facts.find(e.name);
-    if (f != v->facts.end() && f->second.h) w += e.shape[0] * f->second.kp * 2;
+    if (f != v->facts.end() && f->second.h) w += (e.shape[0] + 63) / 64 * 64 * f->second.kp * 2;
   }
   if (v->pw) w += (int64_t)kVisD * 768 * 4;
   for (auto& kv : v->bufs) s += (int64_t)kv.second.bytes;

@@ -21,6 +21,7 @@
 #include "exn_common.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace exn {
 
@@ -44,18 +45,16 @@ __device__ __forceinline__ void wait_dma_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// four values, already scaled, into their hi and lo halves.  The values pass through an empty asm:
-// where V is a product, the compiler would otherwise round it to fp16 in one step for the stored
-// hi (v_fma_mixlo_f16) and in two for the one that lo is taken from, and on a tie they differ.
-__device__ __forceinline__ void split4(const f32x4 x, u32x2& hi, u32x2& lo) {
-  float v[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    v[e] = x[e];
-    asm("" : "+v"(v[e]));
-  }
-  hi = u32x2{pack_f16x2(v[0], v[1]), pack_f16x2(v[2], v[3])};
-  lo = u32x2{pack_f16x2(v[0] - f16_lo(hi[0]), v[1] - f16_hi(hi[0])), pack_f16x2(v[2] - f16_lo(hi[1]), v[3] - f16_hi(hi[1]))};
+// four values, already scaled, into their hi and lo halves.  The packed hi passes through an empty
+// asm, so that lo is taken from the very bits stored: the compiler would otherwise convert twice,
+// and where V is a product round once in one step (v_fma_mixlo_f16) and once in two, which differ on
+// a tie.  The difference is one v_fma_mix_f32 a value.
+__device__ __forceinline__ void split4(const f32x4 v, u32x2& hi, u32x2& lo) {
+  uint32_t h0 = pack_f16x2(v[0], v[1]), h1 = pack_f16x2(v[2], v[3]);
+  asm("" : "+v"(h0), "+v"(h1));
+  hi = u32x2{h0, h1};
+  lo = u32x2{pack_f16x2(__builtin_fmaf(f16_lo(h0), -1.f, v[0]), __builtin_fmaf(f16_hi(h0), -1.f, v[1])),
+             pack_f16x2(__builtin_fmaf(f16_lo(h1), -1.f, v[2]), __builtin_fmaf(f16_hi(h1), -1.f, v[3]))};
 }
 
 // where column K (a multiple of 4) of a split row lies, in halves; its lo part is 32 further
@@ -63,55 +62,70 @@ __device__ __forceinline__ int split_at(int k) { return (k >> 5) * 64 + (k & 31)
 
 // --- the weights -----------------------------------------------------------------------------
 
+// N fp16 (or bf16) values as fp32, subnormals, infinities and NaNs kept
+__global__ void k_vis_widen(int64_t n, const uint16_t* __restrict__ x, int bf16, float* __restrict__ y) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) y[i] = bf16 ? bf16_to_f32(x[i]) : f16_to_f32(x[i]);
+}
+
+hipError_t vis_widen(hipStream_t s, int64_t n, const uint16_t* x, int bf16, float* y) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_vis_widen, dim3(sgrid(n, 256)), dim3(256), 0, s, n, x, bf16, y);
+  return hipGetLastError();
+}
+
 // rec[0] = the bits of the largest |x|, rec[1] those of the largest row's sum of squares (NaNs
 // compare above every number, so a bound made from a tensor that holds one is not finite)
 __global__ void __launch_bounds__(256)
-k_vis_stats(int64_t cols, const float* __restrict__ x, uint32_t* __restrict__ rec) {
-  __shared__ float rm[4], rs[4];
-  const float* r = x + (int64_t)blockIdx.x * cols;
-  uint32_t mb = 0u;
-  float s = 0.f;
-  for (int64_t i = threadIdx.x; i < cols; i += 256) {
-    const float v = r[i];
-    mb = max(mb, __float_as_uint(fabsf(v)));
-    s += v * v;
+k_vis_stats(int64_t rows, int64_t cols, const float* __restrict__ x, uint32_t* __restrict__ rec) {
+  // a wave a row; one pair of atomics a workgroup (one a row took 100 us for 4304 rows)
+  __shared__ uint32_t rm[4], rs[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t mb = 0u, sb = 0u;
+  for (int64_t row = (int64_t)blockIdx.x * 4 + wave; row < rows; row += (int64_t)gridDim.x * 4) {
+    const float* r = x + row * cols;
+    float s = 0.f;
+    for (int64_t i = lane; i < cols; i += 64) {
+      const float v = r[i];
+      mb = max(mb, __float_as_uint(fabsf(v)));
+      s += v * v;
+    }
+    sb = max(sb, __float_as_uint(fabsf(wave_sum(s))));
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mb = max(mb, (uint32_t)__shfl_xor((int)mb, o, 64));
-  s = wave_sum(s);
-  const int wave = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) {
-    rm[wave] = __uint_as_float(mb);
-    rs[wave] = s;
+  if (lane == 0) {
+    rm[wave] = mb;
+    rs[wave] = sb;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-#pragma unroll
-    for (int w = 1; w < 4; ++w) {
-      mb = max(mb, __float_as_uint(rm[w]));
-      s += rs[w];
-    }
-    atomicMax(rec, mb);
-    atomicMax(rec + 1, __float_as_uint(fabsf(s)));
+    atomicMax(rec, max(max(rm[0], rm[1]), max(rm[2], rm[3])));
+    atomicMax(rec + 1, max(max(rs[0], rs[1]), max(rs[2], rs[3])));
   }
 }
 
 hipError_t vis_stats(hipStream_t s, int64_t rows, int64_t cols, const float* x, uint32_t* rec) {
   if (rows <= 0 || cols <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_vis_stats, dim3((unsigned)rows), dim3(256), 0, s, cols, x, rec);
+  hipLaunchKernelGGL(k_vis_stats, dim3((unsigned)std::min<int64_t>((rows + 3) / 4, 512)), dim3(256), 0, s, rows, cols, x,
+                     rec);
   return hipGetLastError();
 }
 
-// rows of K floats, times SCALE, as fp16 rows of KP (zeros past K); *INEXACT set when one changes
+// rows of K floats, times SCALE, as fp16 in the product's order: for each 32 columns of KP, the NP
+// rows' 64 bytes (rows past ROWS and columns past K zero), so that a tile's k-step is one run of
+// whole cache lines; *INEXACT set when a value changes
 __global__ void __launch_bounds__(256)
-k_vis_pack(int K, int KP, float scale, const float* __restrict__ x, uint16_t* __restrict__ y, uint32_t* inexact) {
-  const float* r = x + (int64_t)blockIdx.x * K;
+k_vis_pack(int rows, int K, int KP, float scale, const float* __restrict__ x, uint16_t* __restrict__ y,
+           uint32_t* inexact) {
+  const int row = blockIdx.x, NP = gridDim.x;
+  const float* r = x + (int64_t)row * K;
   bool bad = false;
   for (int i = threadIdx.x; i < KP; i += 256) {
-    const float v = i < K ? r[i] * scale : 0.f;
+    const float v = i < K && row < rows ? r[i] * scale : 0.f;
     const _Float16 h = (_Float16)v;
     bad |= (float)h != v;
-    y[(int64_t)blockIdx.x * KP + i] = __builtin_bit_cast(uint16_t, h);
+    y[((int64_t)(i >> 5) * NP + row) * 32 + (i & 31)] = __builtin_bit_cast(uint16_t, h);
   }
   if (bad) atomicOr(inexact, 1u);
 }
@@ -119,7 +133,8 @@ k_vis_pack(int K, int KP, float scale, const float* __restrict__ x, uint16_t* __
 hipError_t vis_pack(hipStream_t s, int64_t rows, int K, int KP, float scale, const float* x, uint16_t* y,
                     uint32_t* inexact) {
   if (rows <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_vis_pack, dim3((unsigned)rows), dim3(256), 0, s, K, KP, scale, x, y, inexact);
+  hipLaunchKernelGGL(k_vis_pack, dim3((unsigned)((rows + 63) / 64 * 64)), dim3(256), 0, s, (int)rows, K, KP, scale, x, y,
+                     inexact);
   return hipGetLastError();
 }
 
@@ -214,21 +229,27 @@ __device__ __forceinline__ float gelu_sig(float v) {
 // Y^T tiles: the W rows are the MFMAs' A operand and the X rows their B, so that a lane ends with
 // 4 consecutive output columns of one row (v_mfma_f32_16x16x32_f16, D: lane l holds X row l % 16,
 // W rows 4 (l / 16) + e).  Workgroup tiles of BM x BN, WMW x WNW waves of (16 MI) x (16 NI); a
-// k-step of BK moves the tile's X rows (4 BK bytes, hi and lo) and W rows (2 BK bytes) to LDS by
-// DMA, NS stages, the step's DMA going out NS - 1 steps ahead.  A row's 16-byte chunk c is stored
-// at c ^ (row / (256 / row bytes)), so that the 16 rows a fragment read touches at one chunk fall
-// in distinct banks.  Every W fragment meets two X fragments.  OUT 0: fp32 + bias (+ R); 1: GELU
-// (ACT 1 tanh, 2 erf), times OSCALE, into split rows of LDY; 2: fp32 sums of workgroup z's k-steps
-// (split K) at z M N.
+// k-step of 32 moves the tile's X rows (128 bytes, hi and lo) and W rows (64 bytes) to LDS by DMA,
+// NS stages.  A row's 16-byte chunk c is stored at c ^ (row / (256 / row bytes)), so that the 16
+// rows a fragment read touches at one chunk fall in distinct banks.  Every W fragment meets two X
+// fragments.  A step is two halves over the wave's W fragments, so that reads, DMA and MFMAs
+// overlap with one barrier a step and no second set of fragments:
+//   half 1: the X fragments against W's first NA, while W's others are read;
+//   barrier: every read of the step's stage is done, and the next step's DMA has landed;
+//   the DMA of step + NS into the stage just freed;
+//   half 2: the X fragments against W's others, while the next step's first NA W fragments and,
+//   each once its last MFMA is out, its X fragments are read.
+// OUT 0: fp32 + bias (+ R); 1: GELU (ACT 1 tanh, 2 erf), times OSCALE, into split rows of LDY; 2:
+// fp32 sums of workgroup z's k-steps (split K) at z M N.
 enum { VS_F32 = 0, VS_SPLIT = 1, VS_PART = 2 };
-template <int WMW, int WNW, int MI, int NI, int BK, int NS, int OUT, int ACT>
+template <int WMW, int WNW, int MI, int NI, int NS, int OUT, int ACT>
 __global__ void __launch_bounds__(WMW * WNW * 64)
 k_vis_gemm_s(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W, const float* __restrict__ bias,
              const float* R, void* Y, int M, int N, int KP, float descale, float oscale, int ldy) {
-  constexpr int NW = WMW * WNW, BM = WMW * MI * 16, BN = WNW * NI * 16;
-  constexpr int XR = 4 * BK, WR = 2 * BK, XC = XR / 16, WC = WR / 16;   // row bytes, chunks a row
-  constexpr int XS = BM * XR, STAGE = XS + BN * WR, XI = XS / 1024 / NW, WI = BN * WR / 1024 / NW;
-  static_assert(XI * 1024 * NW == XS && WI * 1024 * NW == BN * WR, "whole DMA instructions a wave");
+  constexpr int NW = WMW * WNW, BM = WMW * MI * 16, BN = WNW * NI * 16, NA = (NI + 1) / 2, NB = NI - NA;
+  constexpr int XS = BM * 128, STAGE = XS + BN * 64, XI = XS / 1024, TI = STAGE / 1024;   // DMA instructions a stage
+  constexpr int PER = (TI + NW - 1) / NW, REM = TI % NW;   // a wave's: PER, waves REM and up one less (REM > 0)
+  static_assert(TI * 1024 == STAGE && NB > 0 && XI % NW == 0, "whole DMA instructions, two halves");
   extern __shared__ __align__(1024) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c16 = lane & 15, g = lane >> 4;
@@ -245,70 +266,95 @@ k_vis_gemm_s(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W, con
     bn = in / sz;
   }
   const int tm = bm * BM, tn = bn * BN;
-  const int nk = KP / BK, kt0 = (int)((int64_t)nk * blockIdx.z / gridDim.z),
+  const int nk = KP / 32, kt0 = (int)((int64_t)nk * blockIdx.z / gridDim.z),
             kt1 = (int)((int64_t)nk * (blockIdx.z + 1) / gridDim.z);
   const uint16_t* xb = X + (int64_t)tm * 2 * KP;
-  const uint16_t* wb = W + (int64_t)tn * KP;
-  const uint32_t xext = (uint32_t)((int64_t)min(BM, M - tm) * KP * 4), 
-                 wext = (uint32_t)((int64_t)max(0, min(BN, N - tn)) * KP * 2);
-  auto xswz = [](int r) { return (r / (256 / XR)) % XC; };
-  auto wswz = [](int r) { return (r / (256 / WR)) % WC; };
-  uint32_t xoff[XI], woff[WI];
+  const int NP = (N + 63) / 64 * 64;
+  const uint16_t* wb = W + (int64_t)tn * 32;
+  const uint32_t xext = (uint32_t)((int64_t)min(BM, M - tm) * KP * 4),
+                 wext = (uint32_t)(max(0, min(BN, NP - tn)) * 64);
+  // DMA: a stage is TI runs of 1 KB, wave w takes runs w, w + NW, ..: the first XI are X's (8 rows
+  // each), the others W's (16 rows each)
+  uint32_t off[PER];
 #pragma unroll
-  for (int i = 0; i < XI; ++i) {
-    const int P = 64 * (wave * XI + i) + lane, r = P / XC, c = (P % XC) ^ xswz(r);
-    xoff[i] = (uint32_t)(r * KP * 4 + c * 16);
+  for (int i = 0; i < PER; ++i) {
+    const int p = wave + NW * i;
+    const int rx = 8 * p + (lane >> 3), cx = (lane & 7) ^ ((rx >> 1) & 7);
+    const int rw = 16 * (p - XI) + (lane >> 2), cw = (lane & 3) ^ ((rw >> 2) & 3);
+    off[i] = i < XI / NW ? (uint32_t)(rx * KP * 4 + cx * 16) : (uint32_t)(rw * 64 + cw * 16);
   }
-#pragma unroll
-  for (int i = 0; i < WI; ++i) {
-    const int P = 64 * (wave * WI + i) + lane, r = P / WC, c = (P % WC) ^ wswz(r);
-    woff[i] = (uint32_t)(r * KP * 2 + c * 16);
-  }
-  auto issue = [&](int kt, int st) {
-    uint8_t* base = smem + st * STAGE;
-#pragma unroll
-    for (int i = 0; i < XI; ++i) sdma16(xb, xext, (lds_void*)(base + (wave * XI + i) * 1024), xoff[i], kt * XR);
-#pragma unroll
-    for (int i = 0; i < WI; ++i) sdma16(wb, wext, (lds_void*)(base + XS + (wave * WI + i) * 1024), woff[i], kt * WR);
+  auto issue1 = [&](int kt, int st, int i) {
+    const int p = wave + NW * i;
+    uint8_t* dst = smem + st * STAGE + p * 1024;
+    if (REM && i == PER - 1 && wave >= REM) return;
+    if (i < XI / NW) sdma16(xb, xext, (lds_void*)dst, off[i], kt * 128);
+    else sdma16(wb + (int64_t)kt * NP * 32, wext, (lds_void*)dst, off[i], 0);
   };
-  // a fragment's row c16 of a 16-row block: its chunk c is at 16 (c ^ swz); the swizzle of row
-  // 16 i + c16 is c16's, since 16 rows are whole periods of it
-  const int xs = xswz(c16), ws = wswz(c16);
-  const uint8_t* xrd = smem + (wm + c16) * XR;
-  const uint8_t* wrd = smem + XS + (wn + c16) * WR;
+  // all but the newest KEEP stages' DMA has landed, every LDS read is done, for every wave
+  auto landed = [&](auto keep) {
+    constexpr int KEEP = decltype(keep)::value;
+    if (REM && wave >= REM) wait_dma_barrier<KEEP * (PER - 1)>();
+    else wait_dma_barrier<KEEP * PER>();
+  };
+  const int xs = (c16 >> 1) & 7, ws = (c16 >> 2) & 3;   // a 16-row block's rows: the swizzle is c16's
+  const uint8_t* xrd = smem + (wm + c16) * 128;
+  const uint8_t* wrd = smem + XS + (wn + c16) * 64 + 16 * (g ^ ws);
+  const int xh = 16 * (g ^ xs), xl = 16 * ((4 + g) ^ xs);
   f32x4 acc[MI][NI];
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < NI; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  f16x8 x[MI][2], a[NA], b[NB];
+  // past the end the DMA re-reads the last step, and nothing reads it: every wait counts the same
 #pragma unroll
-  for (int p = 0; p < NS - 1; ++p)
-    if (kt0 + p < kt1) issue(kt0 + p, p);
+  for (int p = 0; p < NS; ++p)
+#pragma unroll
+    for (int i = 0; i < PER; ++i) issue1(min(kt0 + p, kt1 - 1), p, i);
+  landed(std::integral_constant<int, NS - 1>());
+#pragma unroll
+  for (int j = 0; j < NA; ++j) a[j] = *(const f16x8*)(wrd + j * 1024);
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    x[i][0] = *(const f16x8*)(xrd + i * 2048 + xh);
+    x[i][1] = *(const f16x8*)(xrd + i * 2048 + xl);
+  }
   int st = 0;
   for (int kt = kt0; kt < kt1; ++kt) {
-    // step kt's rows are in for every wave, and every wave is done with step kt - 1's stage
-    if (kt + NS - 2 < kt1) wait_dma_barrier<(NS - 2) * (XI + WI)>();
-    else wait_dma_barrier<0>();
-    if (kt + NS - 1 < kt1) issue(kt + NS - 1, st == 0 ? NS - 1 : st - 1);
-    const uint8_t* xr = xrd + st * STAGE;
-    const uint8_t* wr = wrd + st * STAGE;
-    st = st + 1 == NS ? 0 : st + 1;
+    const int nx = st + 1 == NS ? 0 : st + 1, kn = min(kt + NS, kt1 - 1);
 #pragma unroll
-    for (int h = 0; h < BK / 32; ++h) {
-      f16x8 a[NI];
+    for (int j = 0; j < NB; ++j) b[j] = *(const f16x8*)(wrd + st * STAGE + (NA + j) * 1024);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int j = 0; j < NI; ++j) a[j] = *(const f16x8*)(wr + j * 16 * WR + 16 * ((4 * h + g) ^ ws));
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int i = 0; i < MI; ++i) {
-        const f16x8 xh = *(const f16x8*)(xr + i * 16 * XR + 16 * ((8 * h + g) ^ xs));
-        const f16x8 xl = *(const f16x8*)(xr + i * 16 * XR + 16 * ((8 * h + 4 + g) ^ xs));
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int j = 0; j < NI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[j], xh, acc[i][j], 0, 0, 0);
+        for (int j = 0; j < NA; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[j], x[i][u], acc[i][j], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    landed(std::integral_constant<int, NS - 2>());
 #pragma unroll
-        for (int j = 0; j < NI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[j], xl, acc[i][j], 0, 0, 0);
+    for (int j = 0; j < NA; ++j) a[j] = *(const f16x8*)(wrd + nx * STAGE + j * 1024);
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          acc[i][NA + j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[j], x[i][u], acc[i][NA + j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int d = 0; d < PER; ++d)
+          if (d * 2 * MI / PER == 2 * i + u) issue1(kn, st, d);
+        __builtin_amdgcn_sched_barrier(0);
       }
+      x[i][0] = *(const f16x8*)(xrd + nx * STAGE + i * 2048 + xh);
+      x[i][1] = *(const f16x8*)(xrd + nx * STAGE + i * 2048 + xl);
+      __builtin_amdgcn_sched_barrier(0);
     }
+    st = nx;
   }
+  wait_dma_barrier<0>();   // the last DMA has landed before the workgroup's LDS is another's
   {
 #pragma clang fp contract(off)
 #pragma unroll
@@ -348,25 +394,61 @@ k_vis_gemm_s(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W, con
   }
 }
 
-template <int WMW, int WNW, int MI, int NI, int BK, int NS, int OUT, int ACT>
+template <int WMW, int WNW, int MI, int NI, int NS, int OUT, int ACT>
 static hipError_t gemm_s_t(hipStream_t s, const uint16_t* x, const uint16_t* w, const float* bias, const float* r,
                            void* y, int M, int N, int KP, float descale, float oscale, int ldy, int S) {
-  constexpr int BM = WMW * MI * 16, BN = WNW * NI * 16, lds = NS * (BM * 4 + BN * 2) * BK;
-  const void* kern = (const void*)k_vis_gemm_s<WMW, WNW, MI, NI, BK, NS, OUT, ACT>;
+  constexpr int BM = WMW * MI * 16, BN = WNW * NI * 16, lds = NS * (BM * 128 + BN * 64);
+  const void* kern = (const void*)k_vis_gemm_s<WMW, WNW, MI, NI, NS, OUT, ACT>;
   const hipError_t e = ensure_lds(kern, lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((k_vis_gemm_s<WMW, WNW, MI, NI, BK, NS, OUT, ACT>),
+  hipLaunchKernelGGL((k_vis_gemm_s<WMW, WNW, MI, NI, NS, OUT, ACT>),
                      dim3(sgrid(OUT == VS_SPLIT ? ldy : N, BN), sgrid(M, BM), S), dim3(WMW * WNW * 64), lds, s, x, w, bias,
                      r, y, M, N, KP, descale, oscale, ldy);
   return hipGetLastError();
 }
 
+// The tiles, and what a k-step of one costs (us) for a workgroup alone on its CU and for each of
+// several that share one: fitted to K 1152 and 4304 at 80 to 4096 rows.  The 8-wave tiles fill a
+// CU's LDS and run at 82% of the MFMA rate; the small ones, bound by the CU's LDS DMA (about
+// 60 bytes a ns), are for grids that would leave CUs idle.
+struct VisTile {
+  int bm, bn;
+  float alone, shared;
+};
+static const VisTile kVisTiles[] = {{256, 256, 1.06f, 1.06f}, {256, 288, 1.23f, 1.23f}, {128, 144, 0.56f, 0.56f},
+                                    {128, 128, 0.46f, 0.38f}, {64, 128, 0.33f, 0.26f},  {64, 64, 0.20f, 0.18f},
+                                    {32, 64, 0.165f, 0.11f}};
+constexpr int kVisTileCount = sizeof(kVisTiles) / sizeof(kVisTiles[0]);
+
+// the tile of the least cost for S parts of M x N x KP, and that cost
+static int best_tile(int64_t M, int64_t N, int64_t KP, int S, float* cost) {
+  int best = 0;
+  *cost = 1e30f;
+  for (int t = 0; t < kVisTileCount; ++t) {
+    const VisTile& v = kVisTiles[t];
+    const int64_t per_cu = ((int64_t)sgrid(M, v.bm) * sgrid(N, v.bn) * S + 255) / 256;
+    const float c = (float)(KP / 32 / S) * (per_cu == 1 ? v.alone : v.shared * (float)per_cu);
+    if (c < *cost) {
+      *cost = c;
+      best = t;
+    }
+  }
+  return best;
+}
+
 template <int OUT, int ACT>
 static hipError_t gemm_s_tile(hipStream_t s, const uint16_t* x, const uint16_t* w, const float* bias, const float* r,
                               void* y, int M, int N, int KP, float descale, float oscale, int ldy, int S) {
-  if ((int64_t)sgrid(M, 128) * sgrid(N, 128) >= 192)
-    return gemm_s_t<2, 2, 4, 4, 32, 3, OUT, ACT>(s, x, w, bias, r, y, M, N, KP, descale, oscale, ldy, S);
-  return gemm_s_t<2, 2, 2, 2, 64, 3, OUT, ACT>(s, x, w, bias, r, y, M, N, KP, descale, oscale, ldy, S);
+  float cost;
+  switch (best_tile(M, N, KP, S, &cost)) {
+    case 0: return gemm_s_t<4, 2, 4, 8, 3, OUT, ACT>(s, x, w, bias, r, y, M, N, KP, descale, oscale, ldy, S);
+    case 1: return gemm_s_t<4, 2, 4, 9, 3, OUT, ACT>(s, x, w, bias, r, y, M, N, KP, descale, oscale, ldy, S);
+    case 2: return gemm_s_t<4, 1, 2, 9, 5, OUT, ACT>(s, x, w, bias, r, y, M, N, KP, descale, oscale, ldy, S);
+    case 3: return gemm_s_t<2, 2, 4, 4, 3, OUT, ACT>(s, x, w, bias, r, y, M, N, KP, descale, oscale, ldy, S);
+    case 4: return gemm_s_t<2, 2, 2, 4, 4, OUT, ACT>(s, x, w, bias, r, y, M, N, KP, descale, oscale, ldy, S);
+    case 5: return gemm_s_t<2, 2, 2, 2, 4, OUT, ACT>(s, x, w, bias, r, y, M, N, KP, descale, oscale, ldy, S);
+  }
+  return gemm_s_t<2, 2, 1, 2, 6, OUT, ACT>(s, x, w, bias, r, y, M, N, KP, descale, oscale, ldy, S);
 }
 
 static bool gemm_s_ok(const void* x, const void* w, int64_t M, int64_t N, int64_t KP) {
@@ -385,19 +467,28 @@ hipError_t vis_gemm_s(hipStream_t s, const uint16_t* x, const uint16_t* w, const
   return gemm_s_tile<VS_SPLIT, 2>(s, x, w, bias, nullptr, ys, (int)M, (int)N, (int)KP, descale, oscale, (int)ldy, 1);
 }
 
+// S parts cost a k-step's share each, the parts' store and the LayerNorm's reads (8 bytes a value
+// at about 4 TB/s); whole products read and write the residual in the epilogue instead
 int vis_split(int64_t M, int64_t N, int64_t KP) {
-  // 64 x 64 tiles and about 256 workgroups, a part of at least 6 k-steps of 64
-  const int64_t tiles = (int64_t)sgrid(M, 64) * sgrid(N, 64);
-  const int64_t S = std::min<int64_t>(std::min<int64_t>(256 / tiles, KP / 384), 8);
-  return S < 2 ? 1 : (int)S;
+  int best = 1;
+  float least = 1e30f;
+  for (int S = 1; S <= 8 && S <= KP / 192; ++S) {
+    float c;
+    best_tile(M, N, KP, S, &c);
+    c += (float)(M * N) * 2e-6f * (float)S;
+    if (c < least) {
+      least = c;
+      best = S;
+    }
+  }
+  return best;
 }
 
 hipError_t vis_gemm_part(hipStream_t s, const uint16_t* x, const uint16_t* w, float* part, int64_t M, int64_t N,
                          int64_t KP, float descale, int S) {
   if (M <= 0 || N <= 0) return hipSuccess;
   if (!gemm_s_ok(x, w, M, N, KP) || S < 1 || S > KP / 64) return hipErrorInvalidValue;
-  return gemm_s_t<2, 2, 2, 2, 64, 3, VS_PART, 0>(s, x, w, nullptr, nullptr, part, (int)M, (int)N, (int)KP, descale, 0.f, 0,
-                                                S);
+  return gemm_s_tile<VS_PART, 0>(s, x, w, nullptr, nullptr, part, (int)M, (int)N, (int)KP, descale, 0.f, 0, S);
 }
 
 // --- heads, rotary ---------------------------------------------------------------------------
@@ -480,7 +571,8 @@ hipError_t vis_heads_s(hipStream_t s, int n, int np, int heads, const float* qkv
 // Keys past n score -inf; every tile holds a key below n, so the running max is finite.  The
 // output is in v's scale: split rows of KP for attn_out, or (YF) times VDE as fp32 rows.
 #define VS_KT 19456
-#define VS_STAGE (VS_KT + 2 * 9216)
+#define VS_VT 20480   // V^T's hi plane (72 rows of 128 bytes), 1 KB that starts with ones, the lo plane, 1 KB of zeros
+#define VS_LDS (2 * VS_KT + 2 * VS_VT)
 template <int QB>
 __global__ void __launch_bounds__(256, 2)
 k_vis_attend_s(int n, int np, int D, const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
@@ -501,59 +593,82 @@ k_vis_attend_s(int n, int np, int D, const uint16_t* __restrict__ q, const uint1
     qf[b][4] = *(const f16x8*)(qr + (g == 1 ? 136 : 64));
     if (g == 3) qf[b][4] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
   }
-  auto issue = [&](int t, int st) {
+  // the rows of ones and zeros behind each plane (72 .. 79 of the fifth block: their sums are the
+  // probabilities' own)
+  if (tid < 128) {
+    const int st = tid >> 6, i = tid & 63;
+    *(uint32_t*)(smem + 2 * VS_KT + st * VS_VT + 9216 + 4 * i) = 0x3C003C00u;
+    *(uint32_t*)(smem + 2 * VS_KT + st * VS_VT + 10240 + 9216 + 4 * i) = 0u;
+  }
+  const int nt = (n + 63) / 64;
+  auto issue_k = [&](int t) {
     const int key0 = t * 64;
-    uint8_t* base = smem + st * VS_STAGE;
-    const uint32_t kext = (uint32_t)(min(64, n - key0) * (VS_KR * 2)), vext = (uint32_t)((72 * np - key0) * 2);
-    for (int i = wave; i < 37; i += 4) {
-      if (i < 19) {
-        sdma16(kh + (int64_t)key0 * VS_KR, kext, (lds_void*)(base + i * 1024), (uint32_t)(1024 * i + 16 * lane), 0);
-      } else {
-        const int P = 64 * ((i - 19) % 9) + lane, d = P >> 3, c = (P & 7) ^ ((d >> 1) & 7);
-        sdma16(vh + (i < 28 ? 0 : vplane) + key0, vext, (lds_void*)(base + i * 1024), (uint32_t)(d * np * 2 + c * 16), 0);
-      }
-    }
+    uint8_t* base = smem + (t & 1) * VS_KT;
+    const uint32_t kext = (uint32_t)(min(64, n - key0) * (VS_KR * 2));
+#pragma unroll
+    for (int i = 0; i < 5; ++i)
+      if (wave + 4 * i < 19)
+        sdma16(kh + (int64_t)key0 * VS_KR, kext, (lds_void*)(base + (wave + 4 * i) * 1024),
+               (uint32_t)(1024 * (wave + 4 * i) + 16 * lane), 0);
   };
-  float m[QB], l[QB];
-  f32x4 o[5][QB];
+  auto issue_v = [&](int t) {
+    const int key0 = t * 64;
+    uint8_t* base = smem + 2 * VS_KT + (t & 1) * VS_VT;
+    const uint32_t vext = (uint32_t)((72 * np - key0) * 2);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      if (wave + 4 * i < 9) {
+        const int P = 64 * (wave + 4 * i) + lane, d = P >> 3, c = (P & 7) ^ ((d >> 1) & 7);
+        const uint32_t off = (uint32_t)(d * np * 2 + c * 16);
+        sdma16(vh + key0, vext, (lds_void*)(base + (wave + 4 * i) * 1024), off, 0);
+        sdma16(vh + vplane + key0, vext, (lds_void*)(base + 10240 + (wave + 4 * i) * 1024), off, 0);
+      }
+  };
+  float m[QB];
+  f32x4 o[5][QB], s[4][QB];
 #pragma unroll
   for (int b = 0; b < QB; ++b) {
     m[b] = -INFINITY;
-    l[b] = 0.f;
 #pragma unroll
     for (int db = 0; db < 5; ++db) o[db][b] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  // V^T rows 72 .. 79 of the fifth block repeat row 71: their sums are not stored
-  int voff[5];
+  const int e0 = 16 * (g ^ ((c16 >> 1) & 7)), e1 = 16 * ((4 + g) ^ ((c16 >> 1) & 7));
+  const int vr0 = c16 * 128 + e0, vr1 = c16 * 128 + e1;
+  const int vt0 = c16 < 8 ? 8192 + vr0 : 9216, vt1 = c16 < 8 ? 8192 + vr1 : 9216;
+  const int krow = c16 * (VS_KR * 2), km = g < 2 ? 128 : 272;
+  auto read_k = [&](f16x8 (&kf)[5], const uint8_t* kb_, int kb) {
+    const uint8_t* kr = kb_ + krow + kb * (16 * VS_KR * 2);
 #pragma unroll
-  for (int db = 0; db < 5; ++db) voff[db] = min(16 * db + c16, 71);
-  const int nt = (n + 63) / 64;
-  issue(0, 0);
+    for (int c = 0; c < 4; ++c) kf[c] = *(const f16x8*)(kr + (c >> 1) * 144 + (c & 1) * 64 + 16 * g);
+    kf[4] = *(const f16x8*)(kr + km);
+  };
+  auto scores = [&](const f16x8 (&kf)[5], int b) {
+    f32x4 a = {0.f, 0.f, 0.f, 0.f};
+    a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[2], qf[b][0], a, 0, 0, 0);
+    a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[3], qf[b][1], a, 0, 0, 0);
+    a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[0], qf[b][2], a, 0, 0, 0);
+    a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[1], qf[b][3], a, 0, 0, 0);
+    a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[4], qf[b][4], a, 0, 0, 0);
+    a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[0], qf[b][0], a, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[1], qf[b][1], a, 0, 0, 0);
+  };
+  issue_k(0);
+  issue_v(0);
+  if (nt > 1) issue_k(1);
+  wait_dma_barrier<0>();
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) {
+    f16x8 kf[5];
+    read_k(kf, smem, kb);
+#pragma unroll
+    for (int b = 0; b < QB; ++b) s[kb][b] = scores(kf, b);
+  }
   for (int t = 0; t < nt; ++t) {
-    wait_dma_barrier<0>();
-    if (t + 1 < nt) issue(t + 1, (t + 1) & 1);
-    const uint8_t* kb_ = smem + (t & 1) * VS_STAGE;
-    const uint8_t* vb_ = kb_ + VS_KT;
-    f32x4 s[4][QB];
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      const uint8_t* kr = kb_ + (16 * kb + c16) * (VS_KR * 2);
-      f16x8 kf[5];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) kf[c] = *(const f16x8*)(kr + (c >> 1) * 144 + (c & 1) * 64 + 16 * g);
-      kf[4] = *(const f16x8*)(kr + (g < 2 ? 128 : 272));
-#pragma unroll
-      for (int b = 0; b < QB; ++b) {
-        f32x4 a = {0.f, 0.f, 0.f, 0.f};
-        a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[2], qf[b][0], a, 0, 0, 0);
-        a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[3], qf[b][1], a, 0, 0, 0);
-        a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[0], qf[b][2], a, 0, 0, 0);
-        a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[1], qf[b][3], a, 0, 0, 0);
-        a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[4], qf[b][4], a, 0, 0, 0);
-        a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[0], qf[b][0], a, 0, 0, 0);
-        s[kb][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[1], qf[b][1], a, 0, 0, 0);
-      }
-    }
+    // tile t + 1's K and tile t's V are in; every wave is done with tile t's K and tile t - 1's V
+    if (t > 0) wait_dma_barrier<0>();
+    else __syncthreads();
+    if (t + 2 < nt) issue_k(t + 2);
+    if (t + 1 < nt) issue_v(t + 1);
     if (t * 64 + 64 > n) {
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb)
@@ -563,7 +678,12 @@ k_vis_attend_s(int n, int np, int D, const uint16_t* __restrict__ q, const uint1
 #pragma unroll
             for (int b = 0; b < QB; ++b) s[kb][b][e] = -INFINITY;
     }
-    f16x8 ph[2][QB], pl[2][QB];
+    const uint8_t* kn = smem + ((t + 1) & 1) * VS_KT;
+    f16x8 ph[2][QB], pl[2][QB], kf[2][5];
+    float alpha[QB], off[QB];
+    f32x4 sn[4][QB];
+    read_k(kf[0], kn, 0);
+    bool moved = false;
 #pragma unroll
     for (int b = 0; b < QB; ++b) {
       float mx = -INFINITY;
@@ -580,50 +700,55 @@ k_vis_attend_s(int n, int np, int D, const uint16_t* __restrict__ q, const uint1
       // the running max rounded up to a whole number: the exponents' offset and the rescale are
       // then exact, whatever tile a key is in
       const float mn = fmaxf(m[b], ceilf(fmaxf(ma, mb) * sc));
-      // where no query's max moved (most tiles after the first few) there is nothing to rescale
-      if (__any(mn != m[b])) {
-        const float alpha = __builtin_amdgcn_exp2f(m[b] - mn);
-        l[b] *= alpha;
+      alpha[b] = __builtin_amdgcn_exp2f(m[b] - mn);
+      moved |= mn != m[b];
+      m[b] = mn;
+      off[b] = 15.f - mn;
+    }
 #pragma unroll
-        for (int db = 0; db < 5; ++db) o[db][b] = o[db][b] * alpha;
-        m[b] = mn;
-      }
-      const float off = 15.f - mn;
-      float ls = 0.f;
+    for (int kb = 0; kb < 4; ++kb) {
+      if (kb < 3) read_k(kf[(kb + 1) & 1], kn, kb + 1);
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
+      for (int b = 0; b < QB; ++b) {
+        sn[kb][b] = scores(kf[kb & 1], b);
         f32x4 p;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kb][b][e], sc, off));
-          ls += p[e];
-        }
+        for (int e = 0; e < 4; ++e) p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kb][b][e], sc, off[b]));
         u32x2 hi, lo;
         split4(p, hi, lo);
         ((u32x2*)&ph[kb >> 1][b])[kb & 1] = hi;
         ((u32x2*)&pl[kb >> 1][b])[kb & 1] = lo;
       }
-      l[b] += ls;
     }
+    // where no query's max moved (most tiles after the first few) there is nothing to rescale
+    if (__any(moved)) {
+#pragma unroll
+      for (int b = 0; b < QB; ++b)
+#pragma unroll
+        for (int db = 0; db < 5; ++db) o[db][b] = o[db][b] * alpha[b];
+    }
+    const uint8_t* vb_ = smem + 2 * VS_KT + (t & 1) * VS_VT;
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int db = 0; db < 5; ++db) {
-        const uint8_t* vr = vb_ + voff[db] * 128 + 16 * ((4 * u + g) ^ ((voff[db] >> 1) & 7));
-        const f16x8 va = *(const f16x8*)vr, vb = *(const f16x8*)(vr + 9216);
+        const uint8_t* vr = vb_ + (db < 4 ? db * 2048 + (u ? vr1 : vr0) : (u ? vt1 : vt0));
+        const f16x8 va = *(const f16x8*)vr, vb = *(const f16x8*)(vr + 10240);
 #pragma unroll
-        for (int b = 0; b < QB; ++b) {
-          o[db][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vb, ph[u][b], o[db][b], 0, 0, 0);
-          o[db][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pl[u][b], o[db][b], 0, 0, 0);
-          o[db][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, ph[u][b], o[db][b], 0, 0, 0);
-        }
+        for (int b = 0; b < QB; ++b) o[db][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vb, ph[u][b], o[db][b], 0, 0, 0);
+#pragma unroll
+        for (int b = 0; b < QB; ++b) o[db][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pl[u][b], o[db][b], 0, 0, 0);
+#pragma unroll
+        for (int b = 0; b < QB; ++b) o[db][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, ph[u][b], o[db][b], 0, 0, 0);
       }
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int b = 0; b < QB; ++b) s[kb][b] = sn[kb][b];
   }
 #pragma unroll
   for (int b = 0; b < QB; ++b) {
-    float lt = l[b];
-    lt += __shfl_xor(lt, 16, 64);
-    lt += __shfl_xor(lt, 32, 64);
+    const float lt = __shfl(o[4][b][0], 32 + c16, 64);   // row 72
     const int qi = q0 + 16 * b + c16;
     if (qi >= n) continue;
 #pragma unroll
@@ -652,16 +777,17 @@ hipError_t vis_attend_s(hipStream_t s, int n, int np, int heads, const uint16_t*
   if (np % 64 || np < n || np >= n + 64 || (int64_t)np * 144 >= ((int64_t)1 << 31) || (ys && kp != heads * 72))
     return hipErrorInvalidValue;
   const int64_t vplane = (int64_t)heads * 72 * np;
-  // 128 queries a workgroup where that still gives every CU one, else 64
-  const bool two = (int64_t)sgrid(n, 128) * heads >= 256;
+  // 128 queries a workgroup (half the reads of K and V) once the CUs hold more than two of 64 each:
+  // 4096 patches 228 against 269 us, 3072 the same, 2048 70 against 64, 1024 33 against 24
+  const bool two = (int64_t)sgrid(n, 128) * heads > 384;
   const void* kern = two ? (const void*)k_vis_attend_s<2> : (const void*)k_vis_attend_s<1>;
-  const hipError_t e = ensure_lds(kern, 2 * VS_STAGE);
+  const hipError_t e = ensure_lds(kern, VS_LDS);
   if (e != hipSuccess) return e;
   if (two)
-    hipLaunchKernelGGL(k_vis_attend_s<2>, dim3(sgrid(n, 128), heads), dim3(256), 2 * VS_STAGE, s, n, np, heads * 72, q, k,
+    hipLaunchKernelGGL(k_vis_attend_s<2>, dim3(sgrid(n, 128), heads), dim3(256), VS_LDS, s, n, np, heads * 72, q, k,
                        vt, vplane, sc, vde, kp, ys, yf);
   else
-    hipLaunchKernelGGL(k_vis_attend_s<1>, dim3(sgrid(n, 64), heads), dim3(256), 2 * VS_STAGE, s, n, np, heads * 72, q, k,
+    hipLaunchKernelGGL(k_vis_attend_s<1>, dim3(sgrid(n, 64), heads), dim3(256), VS_LDS, s, n, np, heads * 72, q, k,
                        vt, vplane, sc, vde, kp, ys, yf);
   return hipGetLastError();
 }
