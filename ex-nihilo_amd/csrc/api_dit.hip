@@ -835,25 +835,46 @@ static int velocity(exn_dit* d, const float* context, int ptext, const float* la
     HIPCHK(hipMemcpyAsync(d->trace, x, (size_t)(n * EXN_W) * 4, hipMemcpyDeviceToDevice, s));
   HIPCHK(stat(0, 0, x, 0, n * EXN_W));
   float *a32 = nullptr, *h32 = nullptr, *gu32 = nullptr, *ff32 = nullptr;   // the int8 block's fp32 rows
+  int8_t* fq = nullptr;   // and its SwiGLU rows in Q8_0
+  uint16_t* fd = nullptr;
   for (int il = 0; il < d->layers; ++il) {
     Layer& L = d->L[(size_t)il];
     if (int8_ok(L.qkv, n) && int8_ok(L.out, n) && int8_ok(L.gate_up, n) && int8_ok(L.down, n) && L.gate_up->pairs) {
       // the reference's *int8* block (src/cuda-dit.lisp:196-231 with mm at :119-124): each
-      // product's fp32 input quantised, the int8 product to fp32 (QKV: fp16 rows for qkv_prep),
-      // and the elementwise steps apart, as the reference runs them
+      // product's fp32 input quantised and the int8 product to fp32 (QKV: fp16 rows for qkv_prep).
+      // The LayerNorm quantises its own rows, and SwiGLU with the next quantisation and the gated
+      // residuals sit in the products' epilogues: the values of the steps apart, bit for bit, and
+      // 1.2 GB less moved a block at 4096 rows
       if (!a32) {
         TRY(dit_buf(d, "a32", (size_t)(l * EXN_W) * 4, (void**)&a32));
+        TRY(dit_buf(d, "i8f", (size_t)(l * EXN_F), (void**)&fq));
+        TRY(dit_buf(d, "i8fd", (size_t)(l * (EXN_F / 32)) * 2, (void**)&fd));
+      }
+      // the steps run apart where the statistics read the fp32 rows that the fused ones never
+      // write, and where the operands pass the fused products' 32-bit offsets
+      const bool apart = st || n * EXN_F >= ((int64_t)1 << 31);
+      if (apart) {
         TRY(dit_buf(d, "h32", (size_t)(l * EXN_W) * 4, (void**)&h32));
         TRY(dit_buf(d, "gu32", (size_t)(l * 2 * EXN_F) * 4, (void**)&gu32));
         TRY(dit_buf(d, "ff32", (size_t)(l * EXN_F) * 4, (void**)&ff32));
       }
+      auto gated = [&](const int8_t* aq, const uint16_t* ad, const exn_w* W, const float* gate) -> hipError_t {
+        if (!apart)
+          return gemm_w8a8_gate_add(s, aq, ad, n, W->qs, W->d, EXN_W, W->cols, x, EXN_W, n0, p, ms, gate);
+        const hipError_t r = gemm_w8a8(s, aq, ad, n, W->qs, W->d, EXN_W, W->cols, h32, EXN_W, 0);
+        return r == hipSuccess ? gate_add(s, n * EXN_W, EXN_W, n0, p, ms, x, h32, gate) : r;
+      };
+      auto normed = [&](const float* m) -> hipError_t {   // ln_mod's rows in xq, xd
+        if (!apart) return ln_mod_q8(s, (int)n, n0, p, ms, x, EXN_W, m, xq, xd);
+        const hipError_t r = ln_mod(s, (int)n, n0, p, ms, x, EXN_W, m, a32, 0);
+        return r == hipSuccess ? quant_q8(s, a32, 0, EXN_W, n, EXN_W, xq, xd) : r;
+      };
       {
-        ProfScope ps(d, EXN_PROF_LN_MOD, 0, nd * Wd * 8);
-        HIPCHK(ln_mod(s, (int)n, n0, p, ms, x, EXN_W, mod + 0 * EXN_W, a32, 0));
+        ProfScope ps(d, EXN_PROF_LN_MOD, 0, nd * Wd * 5);
+        HIPCHK(normed(mod + 0 * EXN_W));
       }
       {
-        ProfScope ps(d, EXN_PROF_QKV, 2 * nd * 3 * Wd * Wd, nd * Wd * 5 + 3 * Wd * Wd * 1.0625 + nd * 3 * Wd * 2);
-        HIPCHK(quant_q8(s, a32, 0, EXN_W, n, EXN_W, xq, xd));
+        ProfScope ps(d, EXN_PROF_QKV, 2 * nd * 3 * Wd * Wd, nd * Wd + 3 * Wd * Wd * 1.0625 + nd * 3 * Wd * 2);
         HIPCHK(gemm_w8a8(s, xq, xd, n, L.qkv->qs, L.qkv->d, 3 * EXN_W, EXN_W, qkv, 3 * EXN_W, 1));
       }
       {
@@ -865,26 +886,27 @@ static int velocity(exn_dit* d, const float* context, int ptext, const float* la
         HIPCHK(attend(s, q, d->kc[(size_t)il], d->vt[(size_t)il], a32, (int)n, n0, p, (int)l, d->lcap, b0, b1, 1.f, 1));
       }
       {
-        ProfScope ps(d, EXN_PROF_OUT, 2 * nd * Wd * Wd, nd * Wd * 5 + Wd * Wd * 1.0625 + nd * Wd * 4 * 4);
+        ProfScope ps(d, EXN_PROF_OUT, 2 * nd * Wd * Wd, nd * Wd * 5 + Wd * Wd * 1.0625 + nd * Wd * 8);
         HIPCHK(quant_q8(s, a32, 0, EXN_W, n, EXN_W, xq, xd));
-        HIPCHK(gemm_w8a8(s, xq, xd, n, L.out->qs, L.out->d, EXN_W, EXN_W, h32, EXN_W, 0));
-        HIPCHK(gate_add(s, n * EXN_W, EXN_W, n0, p, ms, x, h32, mod + 1 * EXN_W));
+        HIPCHK(gated(xq, xd, L.out, mod + 1 * EXN_W));
       }
       {
-        ProfScope ps(d, EXN_PROF_LN_MOD, 0, nd * Wd * 8);
-        HIPCHK(ln_mod(s, (int)n, n0, p, ms, x, EXN_W, mod + 2 * EXN_W, a32, 0));
+        ProfScope ps(d, EXN_PROF_LN_MOD, 0, nd * Wd * 5);
+        HIPCHK(normed(mod + 2 * EXN_W));
       }
       {
-        ProfScope ps(d, EXN_PROF_GATE_UP, 2 * nd * Wd * 2 * Fd, nd * Wd * 5 + 2 * Fd * Wd * 1.0625 + nd * Fd * 16);
-        HIPCHK(quant_q8(s, a32, 0, EXN_W, n, EXN_W, xq, xd));
-        HIPCHK(gemm_w8a8(s, xq, xd, n, L.gate_up->qs, L.gate_up->d, 2 * EXN_F, EXN_W, gu32, 2 * EXN_F, 0));
-        HIPCHK(swiglu_pairs(s, n, EXN_F, gu32, ff32));
+        ProfScope ps(d, EXN_PROF_GATE_UP, 2 * nd * Wd * 2 * Fd, nd * Wd + 2 * Fd * Wd * 1.0625 + nd * Fd);
+        if (!apart) {
+          HIPCHK(gemm_w8a8_swiglu(s, xq, xd, n, L.gate_up->qs, L.gate_up->d, 2 * EXN_F, EXN_W, fq, fd));
+        } else {
+          HIPCHK(gemm_w8a8(s, xq, xd, n, L.gate_up->qs, L.gate_up->d, 2 * EXN_F, EXN_W, gu32, 2 * EXN_F, 0));
+          HIPCHK(swiglu_pairs(s, n, EXN_F, gu32, ff32));
+          HIPCHK(quant_q8(s, ff32, 0, EXN_F, n, EXN_F, fq, fd));
+        }
       }
       {
-        ProfScope ps(d, EXN_PROF_DOWN, 2 * nd * Fd * Wd, nd * Fd * 5 + Fd * Wd * 1.0625 + nd * Wd * 4 * 4);
-        HIPCHK(quant_q8(s, ff32, 0, EXN_F, n, EXN_F, xq, xd));
-        HIPCHK(gemm_w8a8(s, xq, xd, n, L.down->qs, L.down->d, EXN_W, EXN_F, h32, EXN_W, 0));
-        HIPCHK(gate_add(s, n * EXN_W, EXN_W, n0, p, ms, x, h32, mod + 3 * EXN_W));
+        ProfScope ps(d, EXN_PROF_DOWN, 2 * nd * Fd * Wd, nd * Fd + Fd * Wd * 1.0625 + nd * Wd * 8);
+        HIPCHK(gated(fq, fd, L.down, mod + 3 * EXN_W));
       }
       HIPCHK(stat(il + 1, 0, x, 0, n * EXN_W));
       HIPCHK(stat(il + 1, 1, a32, 0, n * EXN_W));

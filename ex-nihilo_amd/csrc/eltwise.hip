@@ -29,10 +29,13 @@ __device__ __forceinline__ float block_sum256(float v, float* red) {
   return red[0] + red[1] + red[2] + red[3];
 }
 
-// one block a row of 4096: 16 values a thread, kept in registers between the passes
+// one block a row of 4096: 16 values a thread, kept in registers between the passes.  OUT: fp32
+// rows, bf16 rows, or Q8_0 (codes OUT, scales D; 8 lanes hold a block's 32 values)
+enum { LN_F32 = 0, LN_BF16 = 1, LN_Q8 = 2 };
+template <int OUT>
 __global__ void __launch_bounds__(256)
 k_ln_mod(int n, int n0, int p, int mstride, const float* __restrict__ x, int64_t ldx, const float* __restrict__ mod,
-         void* __restrict__ out, int out_bf16) {
+         void* __restrict__ out, uint16_t* __restrict__ d) {
   __shared__ float red[8];
   const int t = blockIdx.x, tid = threadIdx.x;
   const float* r = x + (int64_t)t * ldx;
@@ -60,10 +63,23 @@ k_ln_mod(int n, int n0, int p, int mstride, const float* __restrict__ x, int64_t
     f32x4 o;
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = v[i][e] * inv * (1.f + mv[e]);
-    if (out_bf16) {
+    if constexpr (OUT == LN_BF16) {
       *(u32x2*)((uint16_t*)out + (int64_t)t * 4096 + c) = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
-    } else {
+    } else if constexpr (OUT == LN_F32) {
       *(f32x4*)((float*)out + (int64_t)t * 4096 + c) = o;
+    } else {
+      float mx = fmaxf(fmaxf(fabsf(o[0]), fabsf(o[1])), fmaxf(fabsf(o[2]), fabsf(o[3])));
+      mx = fmaxf(mx, dpp_f<0xB1>(mx));
+      mx = fmaxf(mx, dpp_f<0x4E>(mx));
+      mx = fmaxf(mx, dpp_f<0x141>(mx));
+      const float dd = __fdiv_rn(mx, 127.f);
+      uint32_t w = 0u;
+      if (mx != 0.f) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w |= (uint32_t)((int)roundf(__fdiv_rn(o[e], dd)) & 0xFF) << (8 * e);
+      }
+      *(uint32_t*)((int8_t*)out + (int64_t)t * 4096 + c) = w;
+      if ((tid & 7) == 0) d[(int64_t)t * 128 + (c >> 5)] = __builtin_bit_cast(uint16_t, (_Float16)dd);
     }
   }
 }
@@ -71,7 +87,17 @@ k_ln_mod(int n, int n0, int p, int mstride, const float* __restrict__ x, int64_t
 hipError_t ln_mod(hipStream_t s, int n, int n0, int p, int mstride, const float* x, int64_t ldx, const float* mod,
                   void* out, int out_bf16) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_ln_mod, dim3(n), dim3(256), 0, s, n, n0, p, mstride, x, ldx, mod, out, out_bf16);
+  if (out_bf16)
+    hipLaunchKernelGGL(k_ln_mod<LN_BF16>, dim3(n), dim3(256), 0, s, n, n0, p, mstride, x, ldx, mod, out, nullptr);
+  else
+    hipLaunchKernelGGL(k_ln_mod<LN_F32>, dim3(n), dim3(256), 0, s, n, n0, p, mstride, x, ldx, mod, out, nullptr);
+  return hipGetLastError();
+}
+
+hipError_t ln_mod_q8(hipStream_t s, int n, int n0, int p, int mstride, const float* x, int64_t ldx, const float* mod,
+                     int8_t* q, uint16_t* d) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_ln_mod<LN_Q8>, dim3(n), dim3(256), 0, s, n, n0, p, mstride, x, ldx, mod, q, d);
   return hipGetLastError();
 }
 

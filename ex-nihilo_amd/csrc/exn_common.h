@@ -267,6 +267,17 @@ hipError_t quant_q8(hipStream_t s, const void* x, int xbf16, int64_t ldx, int64_
                     uint16_t* d);
 hipError_t gemm_w8a8(hipStream_t s, const int8_t* xq, const uint16_t* xd, int64_t M, const int8_t* wq,
                      const uint16_t* wd, int64_t N, int64_t K, void* y, int64_t ldy, int f16out);
+// ... with what follows it in the block fused, hipErrorNotSupported where shapes or alignments do
+// not fit: x += tanh(gate) y (gate_add), and SwiGLU of gates and ups interleaved by 32
+// (swiglu_pairs) quantised again (quant_q8) into Q, D.  The same values bit for bit
+hipError_t gemm_w8a8_gate_add(hipStream_t s, const int8_t* xq, const uint16_t* xd, int64_t M, const int8_t* wq,
+                              const uint16_t* wd, int64_t N, int64_t K, float* x, int64_t ldx, int n0, int p, int mstride,
+                              const float* gate);
+hipError_t gemm_w8a8_swiglu(hipStream_t s, const int8_t* xq, const uint16_t* xd, int64_t M, const int8_t* wq,
+                            const uint16_t* wd, int64_t N, int64_t K, int8_t* q, uint16_t* d);
+// ln_mod (width 4096) straight into Q8_0 (quant_q8's values of the fp32 rows)
+hipError_t ln_mod_q8(hipStream_t s, int n, int n0, int p, int mstride, const float* x, int64_t ldx, const float* mod,
+                     int8_t* q, uint16_t* d);
 // Q [32][QLD][128] (QLD 0: N), queries Q0 .. Q0 + N - 1 over keys 0 .. L - 1 under xa_lim
 hipError_t attend(hipStream_t s, const uint16_t* q, const uint16_t* k, const uint16_t* vt, void* out,
                   int n, int q0, int p, int l, int64_t lcap, int b0, int b1, float scale, int of32 = 0,

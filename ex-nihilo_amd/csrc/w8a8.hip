@@ -9,14 +9,30 @@
 //            in fp32, blocks in order: the scale product rounded, the fused multiply-add
 //            rounded once (ggml's sum += d * sumi as its CUDA compiler fuses it).
 //
-// On gfx950 the per-32 rescale, not the int8 MFMA, bounds the product: every 16x16x32 MFMA
-// leaves 4 int32 sums a lane that each take a conversion, the scale product and a fused
-// multiply-add.  k_gemm_w8a8_dma (below) is the product the model runs; k_gemm_w8a8, whose
-// operands come straight from L2 into the MFMA registers, takes the shapes the DMA path does
-// not (K not a multiple of 64, unaligned rows).
+// On gfx950 the per-32 rescale, not the int8 MFMA, bounds the product: every 32 x 32 x 32 block
+// leaves 16 int32 sums a lane that each take a conversion, a scale product and a fused
+// multiply-add.  k_gemm_w8a8_dma (below) is the product the model runs: its scale products come
+// from a second MFMA (the outer product of the block's row and column scales, exact: two fp16
+// factors fit fp32), which leaves two VALU instructions a sum.  gate_up at 4096 rows (824 GOP):
+// 1329 us with the scale products on the SIMD lanes over 16 x 16 x 32 MFMAs, 1306 with them on
+// 4 x 4 x 4 MFMAs, 1177 as it is; the cycles fell by 23%, the clock by 14% (the chip's power).
+// k_gemm_w8a8, whose operands come straight from L2 into the MFMA registers, takes the shapes the
+// DMA path does not (K not a multiple of 64, unaligned rows).
 #include "exn_common.h"
 
 namespace exn {
+
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
+
+// the fused epilogues' operands: the gates (row past the prefix, MSTRIDE on: within it), the
+// sequence row of output row 0 and the prefix; the output's codes and scales
+struct W8Epi {
+  const float* gate;
+  int n0, p, mstride;
+  int8_t* q;
+  uint16_t* d;
+};
 
 // rows of K values (fp32, or bf16 when XBF16; ldx apart) to Q8_0: codes [n][K], scales [n][K/32]
 // fp16.  4 lanes a block, 8 values a lane.
@@ -207,21 +223,41 @@ __device__ __forceinline__ void dma4(const void* base, uint32_t extent, lds_void
 
 // The same product with its operands moved HBM/L2 -> LDS by the DMA path, NS stages of a chunk
 // (2 blocks: 64 bytes of K) ahead (3 stages, 51 KB: three workgroups a CU; 4 stages, two
-// workgroups, ran 17% slower, and loads straight from L2 into registers twice as slow again): per stage the tile's 128 code rows of X and of W (8 KB each,
-// row r's 16-byte chunk c stored at c ^ (r / 4 % 4), so the fragment reads are conflict-free)
-// and their fp16 scales of the two blocks (512 bytes each).  A wave's DMA a chunk is five
-// instructions (2 X, 2 W, 1 scales), so waiting for chunk c while the NS - 2 after it are out
-// is vmcnt(5 (NS - 2)).  Rows past M or N read as zeros (the buffer extents) and are not
-// stored.  K a multiple of 64, ldx-free: X and W rows K bytes apart.
+// workgroups, ran 17% slower, and loads straight from L2 into registers twice as slow again): per
+// stage the tile's 128 code rows of X and of W (8 KB each, row r's 16-byte chunk c stored at
+// c ^ (r / 4 % 4), so the fragment reads are conflict-free) and their fp16 scales of the two
+// blocks (512 bytes each).  A wave's DMA a chunk is five instructions (2 X, 2 W, 1 scales), so
+// waiting for chunk c while the NS - 2 after it are out is vmcnt(5 (NS - 2)).  A wave's 64 x 64
+// are 2 x 2 of v_mfma_i32_32x32x32_i8 (A: lane l holds row l % 32, k = 16 (l / 32) .. +15 of the
+// block; D: lane l holds column l % 32, rows 8 (r / 4) + 4 (l / 32) + r % 4), each beside a
+// v_mfma_f32_32x32x8_f16 of the block's scales.  Rows past M or N read as zeros (the buffer
+// extents) and are not stored.  K a multiple of 64, ldx-free: X and W rows K bytes apart.
+// The epilogues take the block's next steps along: the gated residual (a pass of 200 MB at 4096
+// rows), SwiGLU and the quantisation of its rows (1 GB): the step's int8 block 3.13 -> 2.85 ms.
 #define W8_NS 3
-template <bool F16OUT>
+// what the DMA product does with its sums: fp32 or fp16 rows, the gated residual, or SwiGLU's
+// output in Q8_0 again
+enum { W8_F32 = 0, W8_F16 = 1, W8_GATE_ADD = 2, W8_SWIGLU = 3 };
+
+// the largest of v over the 32 lanes of a half wave, in each of them
+__device__ __forceinline__ float half_max(float v) {
+  v = fmaxf(v, dpp_f<0xB1>(v));
+  v = fmaxf(v, dpp_f<0x4E>(v));
+  v = fmaxf(v, dpp_f<0x141>(v));
+  v = fmaxf(v, dpp_f<0x140>(v));
+  float a = v, b = v;
+  xswap16(a, b);
+  return fmaxf(a, b);
+}
+
+template <int EPI>
 __global__ void __launch_bounds__(256)
 k_gemm_w8a8_dma(const int8_t* __restrict__ xq, const uint16_t* __restrict__ xd, const int8_t* __restrict__ wq,
-                const uint16_t* __restrict__ wd, int64_t M, int64_t N, int64_t K, void* __restrict__ y, int64_t ldy) {
+                const uint16_t* __restrict__ wd, int64_t M, int64_t N, int64_t K, void* __restrict__ y, int64_t ldy,
+                W8Epi ep) {
   // stage s: X codes at s * 17 KB, W codes + 8 KB, X scales + 16 KB, W scales + 16.5 KB
   extern __shared__ __align__(1024) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int c16 = lane & 15, g = lane >> 4;
   const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
   const int64_t tm = (int64_t)blockIdx.y * 128, tn = (int64_t)blockIdx.x * 128;
   const int KB = (int)(K / 32), KC = KB / 2;
@@ -252,26 +288,20 @@ k_gemm_w8a8_dma(const int8_t* __restrict__ xq, const uint16_t* __restrict__ xd, 
     if (wave < 2) dma4(xsbase, xsext, (lds_void*)(st + 16384 + (wave & 1) * 256), soff, c * 4);
     else dma4(wsbase, wsext, (lds_void*)(st + 16896 + (wave & 1) * 256), soff, c * 4);
   };
-  // fragment reads: row tile i (or column tile j) of the wave, block bb of the chunk: LDS row r,
-  // chunk 2 bb + g / 2 at its swizzled place, 8 bytes at 8 (g % 2)
-  int rdx[4], rdw[4];
+  // fragment reads: 32-row tile i (or column tile j) of the wave, block bb of the chunk: LDS row r,
+  // chunk 2 bb + lane / 32 at its swizzled place (tile rows are a multiple of 16 apart, so the
+  // swizzle is the lane's)
+  const int c32 = lane & 31, hi = lane >> 5, fs = (c32 >> 2) & 3;
+  const uint8_t* ard = smem + (wm + c32) * 64;
+  const uint8_t* wrd = smem + 8192 + (wn + c32) * 64;
+  const uint32_t live = hi ? 0u : 0xFFFFFFFFu;   // the outer product's first k lies in lanes 0 .. 31
+  const f32x16 fzero = {};
+  const i32x16 izero = {};
+  f32x16 acc[2][2];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int ra = wm + 16 * i + c16, rb = wn + 16 * i + c16;
-    rdx[i] = ra * 64 + 8 * (g & 1) + ((ra >> 2) & 3) * 16;   // chunk index XORed in below
-    rdw[i] = rb * 64 + 8 * (g & 1) + ((rb >> 2) & 3) * 16;
-  }
-  int32x4 zero = {0, 0, 0, 0};
-  f32x4 acc[4][4];
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto frag = [&](const uint8_t* base, int rd, int chunk) {
-    // rd holds row * 64 + 8 (g % 2) + 16 f(row); the place of chunk c is 16 (c ^ f(row))
-    const int f16x = rd & 0x30;   // 16 f(row)
-    return *(const int64_t*)(base + (rd & ~0x30) + ((chunk * 16) ^ f16x));
-  };
+    for (int j = 0; j < 2; ++j) acc[i][j] = fzero;
   const int nc = KC;
   for (int c = 0; c < W8_NS - 1 && c < nc; ++c) issue(c);
   for (int c = 0; c < nc; ++c) {
@@ -283,93 +313,158 @@ k_gemm_w8a8_dma(const int8_t* __restrict__ xq, const uint16_t* __restrict__ xd, 
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (c + W8_NS - 1 < nc) issue(c + W8_NS - 1);
-    const uint8_t* st = smem + (c % W8_NS) * 17408;
+    const int st = (c % W8_NS) * 17408;
+    int32x4 a[2][2], w[2][2];
+    uint32_t dx[2], dw[2];   // both blocks' scales of the lane's row and column
 #pragma unroll
-    for (int bb = 0; bb < 2; ++bb) {
-      int64_t a[4], w[4];
+    for (int i = 0; i < 2; ++i) {
+      dx[i] = *(const uint32_t*)(smem + st + 16384 + (wm + 32 * i + c32) * 4) & live;
+      dw[i] = *(const uint32_t*)(smem + st + 16896 + (wn + 32 * i + c32) * 4) & live;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        a[i] = frag(st, rdx[i], 2 * bb + (g >> 1));
-        w[i] = frag(st + 8192, rdw[i], 2 * bb + (g >> 1));
+      for (int bb = 0; bb < 2; ++bb) {
+        a[bb][i] = *(const int32x4*)(ard + st + i * 2048 + 16 * ((2 * bb + hi) ^ fs));
+        w[bb][i] = *(const int32x4*)(wrd + st + i * 2048 + 16 * ((2 * bb + hi) ^ fs));
       }
-      f32x4 dx[4];
+    }
+    // product u of the chunk's 8: block u / 4, row tile (u / 2) % 2, column tile u % 2.  Each one's
+    // sums and scales go out before the rescale of the one before, which then waits on no MFMA
+    auto sums = [&](int u) {
+      return __builtin_amdgcn_mfma_i32_32x32x32_i8(a[u >> 2][(u >> 1) & 1], w[u >> 2][u & 1], izero, 0, 0, 0);
+    };
+    auto scales = [&](int u) {
+      const uint32_t x = dx[(u >> 1) & 1], y = dw[u & 1];
+      return __builtin_amdgcn_mfma_f32_32x32x8f16(
+          __builtin_bit_cast(f16x4, u32x2{u >> 2 ? x >> 16 : x & 0xFFFFu, 0u}),
+          __builtin_bit_cast(f16x4, u32x2{u >> 2 ? y >> 16 : y & 0xFFFFu, 0u}), fzero, 0, 0, 0);
+    };
+    i32x16 cur = sums(0);
+    f32x16 sc = scales(0);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const u32x4 u = *(const u32x4*)(st + 16384 + (wm + 16 * i + 4 * g) * 4);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) dx[i][r] = f16_to_f32(bb ? u[r] >> 16 : u[r]);
+    for (int u = 0; u < 8; ++u) {
+      i32x16 nxt;
+      f32x16 nsc;
+      if (u < 7) {
+        nxt = sums(u + 1);
+        nsc = scales(u + 1);
       }
-      float dw[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t u = *(const uint32_t*)(st + 16896 + (wn + 16 * j + c16) * 4);
-        dw[j] = f16_to_f32(bb ? u >> 16 : u);
+      for (int r = 0; r < 16; ++r)
+        acc[(u >> 1) & 1][u & 1][r] = __builtin_fmaf((float)cur[r], sc[r], acc[(u >> 1) & 1][u & 1][r]);
+      cur = nxt;
+      sc = nsc;
+    }
+  }
+  if constexpr (EPI == W8_SWIGLU) {
+    // the wave's columns are 32 gates and their 32 ups: one block of the output a row, its codes
+    // through LDS (the stages are free) for 16-byte stores.  The arithmetic of swiglu_pairs and
+    // quant_q8
+    __syncthreads();
+    int8_t* codes = (int8_t*)smem + wave * 2048;
+    const int64_t blk = (tn + wn) >> 6, KBO = N >> 6;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = 32 * i + 8 * (r >> 2) + 4 * hi + (r & 3);
+        const float v = silu_f(acc[i][0][r]) * acc[i][1][r];
+        const float mx = half_max(fabsf(v)), dd = __fdiv_rn(mx, 127.f);
+        codes[row * 32 + c32] = mx != 0.f ? (int8_t)(int)roundf(__fdiv_rn(v, dd)) : (int8_t)0;
+        if (c32 == 0 && tm + wm + row < M)
+          ep.d[(tm + wm + row) * KBO + blk] = __builtin_bit_cast(uint16_t, (_Float16)dd);
       }
-      int32x4 cur[4], nxt[4];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the wave's own codes
+    if (tm + wm + lane < M) {
+      const u32x4* src = (const u32x4*)(codes + lane * 32);
+      u32x4* dst = (u32x4*)(ep.q + (tm + wm + lane) * (N >> 1) + blk * 32);
+      dst[0] = src[0];
+      dst[1] = src[1];
+    }
+    return;
+  }
+  float g0[2], g1[2];   // W8_GATE_ADD: tanh of the columns' gates, past the prefix and within it
+  if constexpr (EPI == W8_GATE_ADD) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) cur[j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a[0], w[j], zero, 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-#pragma clang fp contract(off)   // the scale product rounded on its own, before the fused multiply-add
-        if (i + 1 < 4) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) nxt[j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a[i + 1], w[j], zero, 0, 0, 0);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float sc = dx[i][r] * dw[j];
-            acc[i][j][r] = __builtin_fmaf((float)cur[j][r], sc, acc[i][j][r]);
-          }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) cur[j] = nxt[j];
-      }
+    for (int j = 0; j < 2; ++j) {
+      const int64_t n = min(tn + wn + 32 * j + c32, N - 1);
+      g0[j] = tanh_f(ep.gate[n]);
+      g1[j] = tanh_f(ep.gate[ep.mstride + n]);
     }
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int64_t m = tm + wm + 16 * i + 4 * g + r;
+    for (int r = 0; r < 16; ++r) {
+      const int64_t m = tm + wm + 32 * i + 8 * (r >> 2) + 4 * hi + (r & 3);
       if (m >= M) continue;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int64_t n = tn + wn + 16 * j + c16;
+      for (int j = 0; j < 2; ++j) {
+        const int64_t n = tn + wn + 32 * j + c32;
         if (n >= N) continue;
-        if constexpr (F16OUT)
+        if constexpr (EPI == W8_F16) {
           ((uint16_t*)y)[m * ldy + n] = __builtin_bit_cast(uint16_t, (_Float16)acc[i][j][r]);
-        else
+        } else if constexpr (EPI == W8_GATE_ADD) {
+          float* x = (float*)y + m * ldy + n;
+          *x = *x + (ep.n0 + m < ep.p ? g1[j] : g0[j]) * acc[i][j][r];
+        } else {
           ((float*)y)[m * ldy + n] = acc[i][j][r];
+        }
       }
     }
+}
+
+template <int EPI>
+static hipError_t launch_w8a8(hipStream_t s, const int8_t* xq, const uint16_t* xd, int64_t M, const int8_t* wq,
+                              const uint16_t* wd, int64_t N, int64_t K, void* y, int64_t ldy, const W8Epi& ep) {
+  const size_t shm = W8_NS * 17408;
+  const hipError_t e = ensure_lds((const void*)k_gemm_w8a8_dma<EPI>, (int)shm);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_gemm_w8a8_dma<EPI>, dim3((unsigned)((N + 127) / 128), (unsigned)((M + 127) / 128)), dim3(256), shm,
+                     s, xq, xd, wq, wd, M, N, K, y, ldy, ep);
+  return hipGetLastError();
+}
+
+// the DMA path: 16-byte code chunks and 4-byte scale pairs, buffer extents within 32 bits
+static bool w8a8_dma_ok(const int8_t* xq, const uint16_t* xd, int64_t M, const int8_t* wq, const uint16_t* wd, int64_t N,
+                        int64_t K) {
+  return K > 0 && K % 64 == 0 && ((uintptr_t)xq & 15) == 0 && ((uintptr_t)wq & 15) == 0 && ((uintptr_t)xd & 3) == 0 &&
+         ((uintptr_t)wd & 3) == 0 && M * K < ((int64_t)1 << 31) && N * K < ((int64_t)1 << 31);
+}
+
+hipError_t gemm_w8a8_gate_add(hipStream_t s, const int8_t* xq, const uint16_t* xd, int64_t M, const int8_t* wq,
+                              const uint16_t* wd, int64_t N, int64_t K, float* x, int64_t ldx, int n0, int p, int mstride,
+                              const float* gate) {
+  if (M <= 0 || N <= 0) return hipSuccess;
+  if (!w8a8_dma_ok(xq, xd, M, wq, wd, N, K) || ldx < N) return hipErrorNotSupported;
+  W8Epi ep{};
+  ep.gate = gate;
+  ep.n0 = n0;
+  ep.p = p;
+  ep.mstride = mstride;
+  return launch_w8a8<W8_GATE_ADD>(s, xq, xd, M, wq, wd, N, K, x, ldx, ep);
+}
+
+hipError_t gemm_w8a8_swiglu(hipStream_t s, const int8_t* xq, const uint16_t* xd, int64_t M, const int8_t* wq,
+                            const uint16_t* wd, int64_t N, int64_t K, int8_t* q, uint16_t* d) {
+  if (M <= 0 || N <= 0) return hipSuccess;
+  if (!w8a8_dma_ok(xq, xd, M, wq, wd, N, K) || N % 64 || ((uintptr_t)q & 15)) return hipErrorNotSupported;
+  W8Epi ep{};
+  ep.q = q;
+  ep.d = d;
+  return launch_w8a8<W8_SWIGLU>(s, xq, xd, M, wq, wd, N, K, nullptr, 0, ep);
 }
 
 hipError_t gemm_w8a8(hipStream_t s, const int8_t* xq, const uint16_t* xd, int64_t M, const int8_t* wq,
                      const uint16_t* wd, int64_t N, int64_t K, void* y, int64_t ldy, int f16out) {
   if (M <= 0 || N <= 0) return hipSuccess;
   if (K % 32 || K <= 0 || ((uintptr_t)xq & 7) || ((uintptr_t)wq & 7) || ldy < N) return hipErrorInvalidValue;
+  if (w8a8_dma_ok(xq, xd, M, wq, wd, N, K))
+    return f16out ? launch_w8a8<W8_F16>(s, xq, xd, M, wq, wd, N, K, y, ldy, W8Epi{})
+                  : launch_w8a8<W8_F32>(s, xq, xd, M, wq, wd, N, K, y, ldy, W8Epi{});
   const dim3 grid((unsigned)((N + 127) / 128), (unsigned)((M + 127) / 128));
-  // the DMA path: 16-byte code chunks and 4-byte scale pairs, buffer extents within 32 bits
-  const bool dma_ok = K % 64 == 0 && ((uintptr_t)xq & 15) == 0 && ((uintptr_t)wq & 15) == 0 &&
-                      ((uintptr_t)xd & 3) == 0 && ((uintptr_t)wd & 3) == 0 && M * K < ((int64_t)1 << 31) &&
-                      N * K < ((int64_t)1 << 31);
-  if (dma_ok) {
-    const size_t shm = W8_NS * 17408;
-    {
-      const hipError_t e = ensure_lds(f16out ? (const void*)k_gemm_w8a8_dma<true> : (const void*)k_gemm_w8a8_dma<false>,
-                                      (int)shm);
-      if (e != hipSuccess) return e;
-    }
-    if (f16out)
-      hipLaunchKernelGGL(k_gemm_w8a8_dma<true>, grid, dim3(256), shm, s, xq, xd, wq, wd, M, N, K, y, ldy);
-    else
-      hipLaunchKernelGGL(k_gemm_w8a8_dma<false>, grid, dim3(256), shm, s, xq, xd, wq, wd, M, N, K, y, ldy);
-  } else if (f16out) {
+  if (f16out)
     hipLaunchKernelGGL(k_gemm_w8a8<true>, grid, dim3(256), 0, s, xq, xd, wq, wd, M, N, K, y, ldy);
-  } else {
+  else
     hipLaunchKernelGGL(k_gemm_w8a8<false>, grid, dim3(256), 0, s, xq, xd, wq, wd, M, N, K, y, ldy);
-  }
   return hipGetLastError();
 }
 

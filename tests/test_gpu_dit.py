@@ -484,6 +484,23 @@ def test_w8a8_mode(ctx):
     d.destroy()
 
 
+@pytest.mark.parametrize("p,h,w", [(9, 1, 7), (40, 11, 13), (131, 16, 16)])
+def test_int8_fused_steps_equal_the_steps_apart(ctx, p, h, w):
+    """The int8 block with the quantisations, SwiGLU and gated residuals in the kernels around them
+    against the same steps run apart (as they are with the statistics on), bit for bit: 16 rows,
+    rows past one and three tiles of 128, the prefix's end inside a tile."""
+    say("int8 fused against apart", p, h, w)
+    d = model(ctx, 2, 23)
+    ctxa, lat = xo.synth_inputs(23, p, h, w)
+    d.w8a8(True)
+    fused = X.dit_velocity(d, ctxa, p, lat, h, w, 0.6)
+    d.stats(True)
+    apart = X.dit_velocity(d, ctxa, p, lat, h, w, 0.6)
+    assert np.isfinite(fused).all() and np.array_equal(fused, apart)
+    d.stats(False)
+    d.destroy()
+
+
 def test_stats_count_a_planted_nan_at_its_block(ctx):
     """*dit-trace*'s numbers (exn_dit_stats): with every value finite they are the largest |x| of
     the stream, the attention's output and the MLP's rows after each block (against the trace's
