@@ -1133,8 +1133,8 @@ static hipError_t launch_w(hipStream_t s, const uint16_t* x, int64_t lda, const 
 }
 
 // --- products over few rows -------------------------------------------------------------
-// A product of at most 256 rows (a prompt's) reads each weight for only that many rows: the
-// weights' stream and (at 256 rows) the MFMAs bound it, and the chip is covered by splitting N
+// A product of 49 to 256 rows (a prompt's; shorter ones: k_gemm_rows below) reads each weight for
+// only that many rows: the weights' stream and (at 256 rows) the MFMAs bound it, and the chip is covered by splitting N
 // finely, not by 256 x 256 tiles with K cut 8 or 16 ways (whose fp32 partial sums then outweigh
 // the weights).  Tiles of MT = 128 WMS rows x NT = 32 (8 / WMS) weight rows, 8 waves of 128 x 32
 // (WMS along M, 8 / WMS along N, two a SIMD), K split over the tile's S workgroups where the
@@ -1344,6 +1344,189 @@ static bool few_fits(const uint16_t* x, int64_t lda, const WOp& w, int64_t M, in
          ea.ldy % 4 == 0 && a16(ea.y) && a16(ea.resid) && a16(ea.gate) && ea.mstride % 4 == 0;
 }
 
+// --- products over very few rows ----------------------------------------------------------
+// A product of at most 48 rows (a short prompt's) is the weights' stream and little else.  k_gemm_few
+// above moves X through LDS a step ahead, one barrier a step, and every step then lasts as long as
+// that DMA (1.1 us for 17 KB of codes); here nothing is shared until the end and no wave waits for
+// another: a workgroup is 64 weight rows, its four waves take every fourth k-step of 64 (K split
+// over S workgroups too where the tiles are fewer than the CUs), each with its W and X fragments
+// straight in registers WD steps ahead, and the four sums meet in LDS, added in the waves' order,
+// before the epilogue.  X's rows come from L2, 16 MI of them (MI KB a wave's slice for W's 2).
+// Operands as k_gemm_few: lane l holds weight row 16 j + l % 16, k = 16 (l / 16) .. +15 of the
+// step, converted to bf16(fp32(d) q); slice kk of the MFMAs sums k = 16 (l / 16) + 8 kk .. +7.
+// Every load is a buffer load whose vector offset the extent covers: rows past M and steps past
+// the wave's last read as zeros.  At 24 rows gate_up (107 MB of codes and scales) took 36.2 us and
+// a split sum of 4.6 there, 28.9 here (3.7 TB/s); to_out and down 20.5 on average, 14.6 here; an
+// encoder of 4 blocks 474 -> 376 us (8 rows 454 -> 328, 48 rows 496 -> 456, 64 rows 509 -> 508).
+template <int EPI, int MI, bool Q8>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_gemm_rows(const uint16_t* __restrict__ X, int64_t lda, const uint16_t* __restrict__ WB,
+            const uint8_t* __restrict__ QT, int64_t M, int64_t N, int64_t K, EpiArgs ea) {
+  constexpr int NI = 4, WD = MI <= 2 ? 4 : 2, LS = 68;   // LS: an LDS row of 64 sums and 4 of padding
+  __shared__ __align__(16) float red[4][16 * MI][LS];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lo = lane & 15, q4 = lane >> 4;
+  const int64_t n0 = (int64_t)blockIdx.x * 64;
+  const int KT = (int)(K / 64), S = gridDim.z, z = blockIdx.z;
+  const int kt0 = (int)((int64_t)KT * z / S), kt1 = (int)((int64_t)KT * (z + 1) / S);
+  const int steps = (kt1 - kt0 + 3) / 4;   // the first wave's; the others' last may be past the end
+  const uint32_t NONE = 0x80000000u;
+  const __amdgpu_buffer_rsrc_t xr =
+      __builtin_amdgcn_make_buffer_rsrc((void*)X, 0, (int)(((M - 1) * lda + K) * 2), 0x00020000);
+  const __amdgpu_buffer_rsrc_t wr =
+      Q8 ? __builtin_amdgcn_make_buffer_rsrc((void*)(QT + (n0 / 256) * (int64_t)KT * QT_CHUNK), 0, KT * QT_CHUNK, 0x00020000)
+         : __builtin_amdgcn_make_buffer_rsrc((void*)(WB + n0 * K), 0, (int)(64 * K * 2), 0x00020000);
+  uint32_t xo[MI], wo[NI], wso[NI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i) xo[i] = 16 * i + lo < M ? (uint32_t)(((16 * i + lo) * lda + 16 * q4) * 2) : NONE;
+#pragma unroll
+  for (int j = 0; j < NI; ++j) {
+    const int row = (int)(n0 % 256) + 16 * j + lo;
+    wo[j] = Q8 ? (uint32_t)(row * 64 + 16 * q4) : (uint32_t)(((16 * j + lo) * K + 16 * q4) * 2);
+    wso[j] = (uint32_t)(QT_SCALES + row * 4);
+  }
+  u32x4 xv[WD][MI][2], wv[WD][NI][Q8 ? 1 : 2];
+  uint32_t wd[WD][NI];
+  auto load = [&](auto uc, int i) {
+    constexpr int u = decltype(uc)::value;
+    const int t = kt0 + wave + 4 * i;
+    const bool live = t < kt1;
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+      const uint32_t o = live ? wo[j] + (uint32_t)t * (Q8 ? QT_CHUNK : 128) : NONE;
+      wv[u][j][0] = __builtin_amdgcn_raw_buffer_load_b128(wr, o, 0, 0);
+      if constexpr (Q8) wd[u][j] = __builtin_amdgcn_raw_buffer_load_b32(wr, live ? wso[j] + (uint32_t)t * QT_CHUNK : NONE, 0, 0);
+      else wv[u][j][Q8 ? 0 : 1] = __builtin_amdgcn_raw_buffer_load_b128(wr, o, 16, 0);
+    }
+#pragma unroll
+    for (int i2 = 0; i2 < MI; ++i2) {
+      const uint32_t o = live && xo[i2] != NONE ? xo[i2] + (uint32_t)t * 128 : NONE;
+      xv[u][i2][0] = __builtin_amdgcn_raw_buffer_load_b128(xr, o, 0, 0);
+      xv[u][i2][1] = __builtin_amdgcn_raw_buffer_load_b128(xr, o, 16, 0);
+    }
+  };
+  f32x4 acc[MI][NI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](auto uc) {
+    constexpr int u = decltype(uc)::value;
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+      const float d = Q8 ? f16_to_f32((wd[u][j] >> (16 * (q4 >> 1))) & 0xFFFFu) : 0.f;
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        u32x4 b;
+        if constexpr (Q8) {
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const uint32_t c = wv[u][j][0][2 * kk + e];
+            b[2 * e] = pack_bf16x2((float)(int8_t)(c & 0xFFu) * d, (float)(int8_t)((c >> 8) & 0xFFu) * d);
+            b[2 * e + 1] = pack_bf16x2((float)(int8_t)((c >> 16) & 0xFFu) * d, (float)(int8_t)(c >> 24) * d);
+          }
+        } else {
+          b = wv[u][j][Q8 ? 0 : kk];
+        }
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xv[u][i][kk]),
+                                                             __builtin_bit_cast(bf16x8, b), acc[i][j], 0, 0, 0);
+      }
+    }
+  };
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, WD == 4 ? 2 : 0>;
+  using I3 = std::integral_constant<int, WD == 4 ? 3 : 1>;
+  load(I0{}, 0);
+  load(I1{}, 1);
+  if constexpr (WD == 4) {
+    load(I2{}, 2);
+    load(I3{}, 3);
+  }
+  for (int i = 0; i < steps; i += WD) {   // whole groups: the steps past the end add zeros
+    compute(I0{});
+    load(I0{}, i + WD);
+    compute(I1{});
+    load(I1{}, i + WD + 1);
+    if constexpr (WD == 4) {
+      compute(I2{});
+      load(I2{}, i + WD + 2);
+      compute(I3{});
+      load(I3{}, i + WD + 3);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[wave][16 * i + 4 * q4 + r][16 * j + lo] = acc[i][j][r];
+  __syncthreads();
+  auto sum = [&](int m, int c) {
+    f32x4 v = *(const f32x4*)&red[0][m][c];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) v += *(const f32x4*)&red[w][m][c];
+    return v;
+  };
+  constexpr int QUADS = EPI == EPI_SWIGLU ? 8 : 16;   // 4-column groups an output row of the tile has
+#pragma unroll
+  for (int it = 0; it < (16 * MI * QUADS + 255) / 256; ++it) {
+    const int id = it * 256 + tid, m = id / QUADS, c = (id % QUADS) * 4;
+    if (m >= M || m >= 16 * MI) continue;
+    const f32x4 v = sum(m, c);
+    if constexpr (EPI == EPI_SWIGLU) {   // columns 0 .. 31 gates, 32 .. 63 their ups
+      const f32x4 u = sum(m, c + 32);
+      *(u32x2*)((uint16_t*)ea.y + m * ea.ldy + n0 / 2 + c) =
+          u32x2{pack_bf16x2(silu_bf16out(v[0]) * u[0], silu_bf16out(v[1]) * u[1]),
+                pack_bf16x2(silu_bf16out(v[2]) * u[2], silu_bf16out(v[3]) * u[3])};
+    } else {
+      const int64_t n = n0 + c;
+      if constexpr (EPI == EPI_PART) {
+        *(f32x4*)((float*)ea.y + ((int64_t)z * M + m) * ea.ldy + n) = v;
+      } else if constexpr (EPI == EPI_F32) {
+        *(f32x4*)((float*)ea.y + m * ea.ldy + n) = v;
+      } else if constexpr (EPI == EPI_BF16) {
+        *(u32x2*)((uint16_t*)ea.y + m * ea.ldy + n) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      } else if constexpr (EPI == EPI_F16) {
+        *(u32x2*)((uint16_t*)ea.y + m * ea.ldy + n) = u32x2{pack_f16x2(v[0], v[1]), pack_f16x2(v[2], v[3])};
+      } else if constexpr (EPI == EPI_GELU_BF16) {
+        *(u32x2*)((uint16_t*)ea.y + m * ea.ldy + n) =
+            u32x2{pack_bf16x2(gelu_tanh_f(v[0]), gelu_tanh_f(v[1])), pack_bf16x2(gelu_tanh_f(v[2]), gelu_tanh_f(v[3]))};
+      } else if constexpr (EPI == EPI_GATE_ADD) {
+        const float* gr = ea.gate + (ea.n0 + m < ea.p ? ea.mstride : 0) + n;
+        f32x4* x = (f32x4*)(ea.resid + m * ea.ldy + n);
+        f32x4 xv4 = *x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) xv4[e] = xv4[e] + tanh_f(gr[e]) * v[e];
+        *x = xv4;
+      }
+    }
+  }
+}
+
+#define ROWS_MAX 48   // at 64 rows (4 row fragments) X's stream from L2 passes W's and nothing is won
+
+// how many workgroups a tile's K is split over: about 1.5 workgroups a CU, each wave at least two
+// steps, at most SMAX
+static int64_t rows_split(int64_t N, int64_t K, int64_t smax) {
+  const int64_t tiles = N / 64;
+  int64_t S = (384 + tiles - 1) / tiles;
+  if (S > K / 64 / 8) S = K / 64 / 8;
+  if (S > smax) S = smax;
+  return S < 1 ? 1 : S;
+}
+
+template <int EPI, bool Q8>
+static hipError_t launch_rows(hipStream_t s, const uint16_t* x, int64_t lda, const WOp& w, int64_t M, int64_t N,
+                              int64_t K, const EpiArgs& ea, int S) {
+  const dim3 grid((unsigned)(N / 64), 1, (unsigned)S);
+  auto kern = M <= 16 ? k_gemm_rows<EPI, 1, Q8> : M <= 32 ? k_gemm_rows<EPI, 2, Q8> : k_gemm_rows<EPI, 3, Q8>;
+  hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, x, lda, w.wb, w.qt, M, N, K, ea);
+  return hipGetLastError();
+}
+
 template <int EPI, bool Q8>
 static hipError_t launch_few(hipStream_t s, const uint16_t* x, int64_t lda, const WOp& w, int64_t M, int64_t N,
                              int64_t K, const EpiArgs& ea, int S) {
@@ -1361,6 +1544,8 @@ static hipError_t launch_few(hipStream_t s, const uint16_t* x, int64_t lda, cons
 template <int EPI>
 static hipError_t launch_few_w(hipStream_t s, const uint16_t* x, int64_t lda, const WOp& w, int64_t M, int64_t N,
                                int64_t K, const EpiArgs& ea, int S) {
+  if (M <= ROWS_MAX)
+    return w.wb ? launch_rows<EPI, false>(s, x, lda, w, M, N, K, ea, S) : launch_rows<EPI, true>(s, x, lda, w, M, N, K, ea, S);
   return w.wb ? launch_few<EPI, false>(s, x, lda, w, M, N, K, ea, S) : launch_few<EPI, true>(s, x, lda, w, M, N, K, ea, S);
 }
 
@@ -1481,7 +1666,7 @@ hipError_t gemm_split_rows(hipStream_t s, const uint16_t* x, int64_t lda, const 
     // at most 256 rows: the few-row tiles, K split so that the tiles' workgroups are about one a
     // CU, each at least 4 k-steps, at most SMAX ways and within PART_CAP
     const int64_t tiles = N / (M > 128 ? 128 : 256);
-    int64_t S = 256 / tiles;
+    int64_t S = M <= ROWS_MAX ? rows_split(N, K, smax) : 256 / tiles;
     if (S > K / 256) S = K / 256;
     if (S > smax) S = smax;
     if (S > part_cap / (M * N)) S = part_cap / (M * N);

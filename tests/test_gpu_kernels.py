@@ -109,6 +109,15 @@ GEMM_CASES = [  # (M, N, K): ragged, the block shapes, proj_out's N = 64, img_in
     (4352, 12288, 4096), (1100, 640, 4096), (513, 128, 128)]
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 256, 256), (16, 256, 768), (17, 512, 1280), (32, 6144, 4096), (33, 256, 12288),
+                                   (48, 1024, 256), (49, 256, 256)])
+def test_very_few_row_products(ctx, M, N, K):
+    """As test_few_row_products at the edges of the kernel for at most 48 rows: one to three row
+    fragments of 16, fewer k-steps than a workgroup's four waves hold (K 256: one each), step counts
+    that end inside a group (768, 1280), and the first row count past it."""
+    test_few_row_products(ctx, M, N, K)
+
+
 @pytest.mark.parametrize("resident", [False, True], ids=["q8_0", "resident_bf16"])
 @pytest.mark.parametrize("M,N,K", GEMM_CASES)
 def test_gemm_q8_bf16(ctx, M, N, K, resident):
