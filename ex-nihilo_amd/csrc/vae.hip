@@ -15,13 +15,18 @@
 // half-size picture and the neighbour's pixel is halved: the nearest x2
 // upsampling (x_up2) folded into the resample convolution's loads.
 //
-// Tiles: 256 pixels x 288 output channels a workgroup where 288 divides the
+// Two kernels: k_conv_halo takes the 3 x 3 convolutions of pictures that 16 x 16 tiles fit, k_conv
+// the others, the 1 x 1 and the stride-2 ones.
+//
+// k_conv's tiles: 256 pixels x 288 output channels a workgroup where 288 divides the
 // width (1152, 576, 288), else 256 x 144 (144 divides every width of the
 // decoder); 8 waves of 144 channels each, v_mfma_f32_16x16x32_bf16; K 64 a
 // step, two LDS stages (72 KB each) at 288, three (50 KB each) at 144.  The
 // epilogue stages each wave's accumulators through LDS 32 pixels at a time,
 // so that bias, residual, DupUp3D and clamp are applied to 16-byte rows.
 #include "exn_common.h"
+
+#include <type_traits>
 
 namespace exn {
 
@@ -60,6 +65,148 @@ struct ConvTile {
   static constexpr int LDS = NST * STAGE > EPI ? NST * STAGE : EPI;
   static_assert(BREM % 8 == 0 && BREM <= 64 && (NW == 8 || LDS <= 80 * 1024), "tile layout");
 };
+
+// The epilogue of a convolution's tile: the wave's accumulators (MI blocks of 16 pixels, block i's
+// rows 4 (l / 16) + r; NJ blocks of 16 channels from n0 + WNC wn), PIX(half, row) the output pixel
+// of row ROW (0 .. 31) of blocks 2 half, 2 half + 1, at least P where there is none.
+template <class T, int BN, int OUT, int GAM, class Pix>
+__device__ __forceinline__ void conv_epilogue(const f32x4 (&acc)[T::MI][T::NJ], uint8_t* smem, const float* bias,
+                                              const VaeEpi& ep, void* Y, int P, int W, int cout, int n0, int wave, int lane,
+                                              int wn, int z, const Pix& pix) {
+  const int lo = lane & 15, q4 = lane >> 4;
+  constexpr bool BIG = T::MI * T::NJ >= 36;   // half the accumulators fill the registers
+  // Through LDS (free now), 32 of the wave's pixels at a time: the wave stages its
+  // 32 x 144 block (row stride 148 floats), then moves it as 16-byte chunks, 4 channels of one
+  // pixel a lane: bias, and the residual or the DupUp3D gather, summed into the staged rows
+  // first, then the stores.
+  float* stg = (float*)smem + wave * (32 * T::LS);
+  const float winv = 1.f / (float)W;
+  const int rsh = OUT == VAE_DUPUP ? __builtin_ctz((unsigned)(cout * ep.ft * 4 / ep.kcin)) : 0;
+#pragma unroll
+  for (int half = 0; half < T::MI / 2; ++half) {
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < T::NJ; ++j)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) stg[(16 * i + 4 * q4 + r) * T::LS + 16 * j + lo] = acc[2 * half + i][j][r];
+    __syncthreads();
+    // NCH chunks a lane (18 at WNC 144), 4 channels of one pixel each, in two passes.  Pass 1
+    // adds bias and the residual or the DupUp3D gather in place in the staging rows, in batches
+    // of 6 chunks (3 at BN 288, where half the accumulators are still live); with no stores
+    // among them the loads of one batch can be in flight while the last is summed.  Pass 2
+    // stores the rows: no load is left to wait for.  (Stores among the loads would make
+    // every batch wait for the stores before it, a round trip to HBM each.)
+    constexpr int CH = BIG ? (OUT == VAE_DUPUP || GAM ? 2 : 3) : (T::NCH < 6 ? T::NCH : 6);
+    static_assert(T::NCH % CH == 0, "whole batches");
+    if constexpr (OUT != VAE_PART) {
+#pragma unroll BIG ? 2 : T::NCH / CH
+      for (int bt = 0; bt < T::NCH / CH; ++bt) {
+        f32x4 v[CH], add[CH];
+#pragma unroll
+        for (int q = 0; q < CH; ++q) {
+          const int k = (bt * CH + q) * 64 + lane, row = k / T::RC, c4 = k - row * T::RC;
+          const int m = pix(half, row), n = n0 + T::WNC * wn + 4 * c4;
+          const int mc = min(m, P - 1), nc = min(n, cout - 4);   // in bounds for the loads either way
+          v[q] = *(const f32x4*)(stg + row * T::LS + 4 * c4);
+          v[q] += *(const f32x4*)(bias + nc);
+          add[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+          if constexpr (OUT == VAE_DUPUP) {
+            // channel c of pixel (yy, xx) adds keep's channel j / rep of pixel (yy/2, xx/2),
+            // j = ((c ft + ft - 1) 2 + yy%2) 2 + xx%2, rep = cout ft 4 / kcin (a power of two)
+            int yy = (int)(((float)mc + 0.5f) * winv);   // mc / W, corrected to exact below
+            yy -= yy * W > mc;
+            yy += (yy + 1) * W <= mc;
+            const int xx = mc - yy * W;
+            const float* kr = ep.keep + (((yy >> 1) * (W >> 1) + (xx >> 1)) * ep.kcin);
+            const int j0 = ((nc * ep.ft + ep.ft - 1) * 2 + (yy & 1)) * 2 + (xx & 1);
+            // keep channel of channel nc + e: (j0 >> rsh) + e * kstep, kstep = kcin / cout (rep
+            // divides 4 ft then).  At kstep 1 that is channels nc .. nc + 3, at kstep 2 channels
+            // 2 nc + d + 0, 2, 4, 6 (d = 0 or 1): one or two aligned 16-byte loads.
+            const int kstep = (4 * ep.ft) >> rsh, k0 = j0 >> rsh;
+            if (kstep == 1 && (4 * ep.ft) % (1 << rsh) == 0) {
+              add[q] = *(const f32x4*)(kr + k0);
+            } else if (kstep == 2 && (4 * ep.ft) % (1 << rsh) == 0) {
+              const f32x4 t0 = *(const f32x4*)(kr + 2 * nc), t1 = *(const f32x4*)(kr + 2 * nc + 4);
+              const int d = k0 - 2 * nc;
+              add[q] = d ? f32x4{t0[1], t0[3], t1[1], t1[3]} : f32x4{t0[0], t0[2], t1[0], t1[2]};
+            } else {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) add[q][e] = kr[(j0 + 4 * ep.ft * e) >> rsh];
+            }
+          } else if constexpr (OUT == VAE_F32 || OUT == VAE_BF16) {
+            if (ep.res) add[q] = *(const f32x4*)(ep.res + (int64_t)mc * cout + nc);
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < CH; ++q) {
+          const int k = (bt * CH + q) * 64 + lane, row = k / T::RC, c4 = k - row * T::RC;
+          *(f32x4*)(stg + row * T::LS + 4 * c4) = v[q] + add[q];
+        }
+      }
+    }
+#pragma unroll BIG ? 3 : 6
+    for (int q = 0; q < T::NCH; ++q) {
+      const int k = q * 64 + lane, row = k / T::RC, c4 = k - row * T::RC;
+      const int m = pix(half, row), n = n0 + T::WNC * wn + 4 * c4;
+      if (m >= P || n >= cout) continue;
+      const int at = m * cout + n;
+      const f32x4 o = *(const f32x4*)(stg + row * T::LS + 4 * c4);
+      if constexpr (OUT == VAE_RMS) {
+      } else if constexpr (OUT == VAE_BF16) {
+        *(u32x2*)((uint16_t*)Y + at) = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+      } else if constexpr (OUT == VAE_PART) {
+        *(f32x4*)((float*)Y + (int64_t)z * P * cout + at) = o;
+      } else if constexpr (OUT == VAE_CLAMP) {
+        f32x4 c;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) c[e] = fminf(1.f, fmaxf(-1.f, o[e]));
+        *(f32x4*)((float*)Y + at) = c;
+      } else {
+        if (OUT != VAE_DUPUP || Y) *(f32x4*)((float*)Y + at) = o;   // DupUp: no fp32 out when Y is null
+        if constexpr (OUT == VAE_F32 || OUT == VAE_DUPUP) {
+          if (ep.y2) *(u32x2*)(ep.y2 + at) = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+        }
+      }
+    }
+    if constexpr (GAM) {
+      static_assert(T::WNC == 144 || T::WNC == 96, "the norm's layout: rows of 144 or 96 a wave");
+      // each staged row's sum of squares: lanes 2r and 2r + 1 take its two halves, then swap; at
+      // BN 288 and 192 the row's other channels are the partner wave's (same pixels)
+      constexpr int HALF4 = T::WNC / 8;   // 4-channel chunks in half a row
+      const int rr = lane >> 1, hh = lane & 1;
+      float ss = 0.f;
+#pragma unroll 3
+      for (int c = 0; c < HALF4; ++c) {
+        const f32x4 t = *(const f32x4*)(stg + rr * T::LS + (T::WNC / 2) * hh + 4 * c);
+        ss += (t[0] * t[0] + t[1] * t[1]) + (t[2] * t[2] + t[3] * t[3]);
+      }
+      ss += dpp_f<0xB1>(ss);   // quad_perm [1, 0, 3, 2]: lane ^ 1
+      if constexpr (T::NWN == 2) {
+        if (hh == 0) stg[rr * T::LS + T::WNC] = ss;
+        __syncthreads();
+        const int partner = wn ? wave - T::NWM : wave + T::NWM;
+        ss += ((const float*)smem + partner * (32 * T::LS))[rr * T::LS + T::WNC];
+      }
+      const float inv = sqrtf((float)cout) / fmaxf(sqrtf(ss), 1e-12f);
+      if (hh == 0) stg[rr * T::LS + T::WNC + 1] = inv;
+      asm volatile("" ::: "memory");
+#pragma unroll 2
+      for (int q = 0; q < T::NCH; ++q) {
+        const int k = q * 64 + lane, row = k / T::RC, c4 = k - row * T::RC;
+        const int m = pix(half, row), n = n0 + T::WNC * wn + 4 * c4;
+        if (m >= P) continue;
+        const f32x4 o = *(const f32x4*)(stg + row * T::LS + 4 * c4), g = *(const f32x4*)(ep.gamma + n);
+        const float iv = stg[row * T::LS + T::WNC + 1];
+        float e[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) e[j] = silu_bf16out(o[j] * iv * g[j]);
+        *(u32x2*)(ep.yr + (int64_t)m * cout + n) = u32x2{pack_bf16x2(e[0], e[1]), pack_bf16x2(e[2], e[3])};
+      }
+    }
+  }
+}
 
 // UP: 0 a 'same' convolution of an H x W picture; 1 the same of the picture nearest-upsampled
 // from H/2 x W/2 (the input); 2 stride 2 over a 2H x 2W input, padded with zeros below and to
@@ -203,137 +350,183 @@ k_conv(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Wt, const fl
   __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0x0 << 8));   // no DMA left in flight
   asm volatile("" ::: "memory");
 
-  // The epilogue through LDS (free now), 32 of the wave's pixels at a time: the wave stages its
-  // 32 x 144 block (row stride 148 floats), then moves it as 16-byte chunks, 4 channels of one
-  // pixel a lane: bias, and the residual or the DupUp3D gather, summed into the staged rows
-  // first, then the stores.
-  float* stg = (float*)smem + wave * (32 * T::LS);
-  const float winv = 1.f / (float)W;
-  const int rsh = OUT == VAE_DUPUP ? __builtin_ctz((unsigned)(cout * ep.ft * 4 / ep.kcin)) : 0;
+  conv_epilogue<T, BN, OUT, GAM>(acc, smem, bias, ep, Y, P, W, cout, n0, wave, lane, wn, z,
+                                 [&](int half, int row) { return m0 + T::WM * wm + 32 * half + row; });
+}
+
+// The 3 x 3 convolutions (UP 0 and 1) whose input lies in LDS once for its nine taps.  k_conv's A
+// tile is gathered tap by tap, and its step then lasts as long as the CU's LDS DMA takes (about 60
+// bytes a ns: 68 KB a step of 1.1 us at 288 channels, 34 KB of 0.5 us twice a CU at 144).  Here a
+// workgroup is 16 x 16 output pixels x BN channels and walks K as chunks of 32 channels, nine taps
+// each: the chunk's 18 x 18 neighbourhood (UP: the half-size picture's 10 x 10) is loaded once, a
+// chunk ahead, and each tap's fragments are read from it at their offset; the weights stream, 64 BN
+// bytes a step, NST stages.  A wave is 4 rows of 16 pixels (MI = 4) x WNC channels.  A neighbourhood
+// pixel is 64 bytes, its 16-byte chunk c at c ^ (pixel / 4 % 4): 16 pixels in a row read at one
+// chunk fall in distinct banks whatever their offset.  A step is four groups of channel blocks, each
+// group's fragments read while the group before is multiplied; before the last one's MFMAs a barrier
+// (every read of the step's stages is done, the next step's weights have landed), and between them
+// the next step's first fragments are read and the DMA of step + NST's weights and, early in a
+// chunk, of the next chunk's neighbourhood goes out.  Channels past C read as zeros.
+// Measured (us, k_conv then this): 288 -> 288 at 512 x 512 508 / 458, 576 -> 576 at 256 x 256 429 /
+// 371, 144 -> 144 at 1024 x 1024 733 / 662 with its fp32 output and 689 / 514 without, upsampling
+// 288 at 1024 x 1024 2011 / 1751, 96 -> 96 at 1024 x 1024 370 / 268; decode 19.6 -> 17.2 ms, encode
+// 5.5 -> 4.8.  What is left runs at about 1.05 PFLOP/s, the chip's power at this mix of reads.
+template <int BN>
+struct HaloTile {
+  static constexpr int WNC = BN % 144 == 0 ? 144 : 96, NJ = WNC / 16, NWN = BN / WNC, NWM = 4, NW = NWM * NWN, MI = 4;
+  static constexpr int LS = WNC + 4, RC = WNC / 4, NCH = 32 * RC / 64;
+  static constexpr int ABYTES = 24576, BBYTES = BN * 64, NST = BN == 288 ? 4 : 3;
+  static constexpr int EPI = NW * 32 * 148 * 4;
+  static constexpr int LDS = 2 * ABYTES + NST * BBYTES > EPI ? 2 * ABYTES + NST * BBYTES : EPI;
+  static constexpr int BFULL = BN * 4 / (64 * NW), BREM = (BN * 4 - 64 * NW * BFULL) / NW, NB_DMA = BFULL + (BREM > 0);
+  static_assert(NW == 8 || LDS <= 80 * 1024, "two workgroups of 4 waves a CU");
+};
+
+template <int BN, int UP, int OUT, int GAM>
+__global__ void __launch_bounds__(HaloTile<BN>::NW * 64, HaloTile<BN>::NW == 4 ? 2 : 1)
+k_conv_halo(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Wt, const float* __restrict__ bias, VaeEpi ep,
+            void* __restrict__ Y, int H, int W, int C, int cout, int Kp) {
+  typedef HaloTile<BN> T;
+  constexpr int HW = UP ? 10 : 18, CHUNKS = HW * HW * 4;   // the neighbourhood's width and 16-byte chunks
+  constexpr int NA_DMA = (CHUNKS + 64 * T::NW - 1) / (64 * T::NW);   // rounds; the last one's spare lanes write zeros
+  static_assert(NA_DMA <= 6 && NA_DMA * T::NW * 1024 <= T::ABYTES, "the neighbourhood's rounds");
+  extern __shared__ __align__(1024) uint8_t smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave % T::NWM, wn = wave / T::NWM, lo = lane & 15, q4 = lane >> 4;
+  const int P = H * W, TW = (W + 15) >> 4;
+  const int ty0 = (blockIdx.x / TW) * 16, tx0 = (blockIdx.x % TW) * 16, n0 = blockIdx.y * BN;
+  // split K (VAE_PART): workgroup z of gridDim.z takes chunks c0 .. c1-1
+  const int NC = (C + 31) / 32, S = gridDim.z, z = blockIdx.z;
+  const int c0 = (int)((int64_t)NC * z / S), c1 = (int)((int64_t)NC * (z + 1) / S);
+  const int Hs = UP ? H >> 1 : H, Ws = UP ? W >> 1 : W;
+  const uint32_t xext = (uint32_t)((int64_t)Hs * Ws * C * 2);
+  const uint16_t* wbase = Wt + (int64_t)n0 * Kp;
+  const uint32_t wext = (uint32_t)((int64_t)max(0, cout - n0) * Kp * 2);
+  // the neighbourhood's rounds: chunk q of it is pixel q / 4's at q % 4 (swizzled); round i of a
+  // wave 64 chunks
+  uint32_t aoff[NA_DMA];   // the byte offset, and in its two lowest bits which 8 of the 32 channels
 #pragma unroll
-  for (int half = 0; half < T::MI / 2; ++half) {
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < T::NJ; ++j)
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) stg[(16 * i + 4 * q4 + r) * T::LS + 16 * j + lo] = acc[2 * half + i][j][r];
-    __syncthreads();
-    // NCH chunks a lane (18 at WNC 144), 4 channels of one pixel each, in two passes.  Pass 1
-    // adds bias and the residual or the DupUp3D gather in place in the staging rows, in batches
-    // of 6 chunks (3 at BN 288, where half the accumulators are still live); with no stores
-    // among them the loads of one batch can be in flight while the last is summed.  Pass 2
-    // stores the rows: no load is left to wait for.  (Stores among the loads would make
-    // every batch wait for the stores before it, a round trip to HBM each.)
-    constexpr int CH = BN == 288 ? (OUT == VAE_DUPUP || GAM ? 2 : 3) : (T::NCH < 6 ? T::NCH : 6);
-    static_assert(T::NCH % CH == 0, "whole batches");
-    if constexpr (OUT != VAE_PART) {
-#pragma unroll BN == 288 ? 2 : T::NCH / CH
-      for (int bt = 0; bt < T::NCH / CH; ++bt) {
-        f32x4 v[CH], add[CH];
-#pragma unroll
-        for (int q = 0; q < CH; ++q) {
-          const int k = (bt * CH + q) * 64 + lane, row = k / T::RC, c4 = k - row * T::RC;
-          const int m = m0 + T::WM * wm + 32 * half + row, n = n0 + T::WNC * wn + 4 * c4;
-          const int mc = min(m, P - 1), nc = min(n, cout - 4);   // in bounds for the loads either way
-          v[q] = *(const f32x4*)(stg + row * T::LS + 4 * c4);
-          v[q] += *(const f32x4*)(bias + nc);
-          add[q] = f32x4{0.f, 0.f, 0.f, 0.f};
-          if constexpr (OUT == VAE_DUPUP) {
-            // channel c of pixel (yy, xx) adds keep's channel j / rep of pixel (yy/2, xx/2),
-            // j = ((c ft + ft - 1) 2 + yy%2) 2 + xx%2, rep = cout ft 4 / kcin (a power of two)
-            int yy = (int)(((float)mc + 0.5f) * winv);   // mc / W, corrected to exact below
-            yy -= yy * W > mc;
-            yy += (yy + 1) * W <= mc;
-            const int xx = mc - yy * W;
-            const float* kr = ep.keep + (((yy >> 1) * (W >> 1) + (xx >> 1)) * ep.kcin);
-            const int j0 = ((nc * ep.ft + ep.ft - 1) * 2 + (yy & 1)) * 2 + (xx & 1);
-            // keep channel of channel nc + e: (j0 >> rsh) + e * kstep, kstep = kcin / cout (rep
-            // divides 4 ft then).  At kstep 1 that is channels nc .. nc + 3, at kstep 2 channels
-            // 2 nc + d + 0, 2, 4, 6 (d = 0 or 1): one or two aligned 16-byte loads.
-            const int kstep = (4 * ep.ft) >> rsh, k0 = j0 >> rsh;
-            if (kstep == 1 && (4 * ep.ft) % (1 << rsh) == 0) {
-              add[q] = *(const f32x4*)(kr + k0);
-            } else if (kstep == 2 && (4 * ep.ft) % (1 << rsh) == 0) {
-              const f32x4 t0 = *(const f32x4*)(kr + 2 * nc), t1 = *(const f32x4*)(kr + 2 * nc + 4);
-              const int d = k0 - 2 * nc;
-              add[q] = d ? f32x4{t0[1], t0[3], t1[1], t1[3]} : f32x4{t0[0], t0[2], t1[0], t1[2]};
-            } else {
-#pragma unroll
-              for (int e = 0; e < 4; ++e) add[q][e] = kr[(j0 + 4 * ep.ft * e) >> rsh];
-            }
-          } else if constexpr (OUT == VAE_F32 || OUT == VAE_BF16) {
-            if (ep.res) add[q] = *(const f32x4*)(ep.res + (int64_t)mc * cout + nc);
-          }
-        }
-#pragma unroll
-        for (int q = 0; q < CH; ++q) {
-          const int k = (bt * CH + q) * 64 + lane, row = k / T::RC, c4 = k - row * T::RC;
-          *(f32x4*)(stg + row * T::LS + 4 * c4) = v[q] + add[q];
-        }
-      }
-    }
-#pragma unroll BN == 288 ? 3 : 6
-    for (int q = 0; q < T::NCH; ++q) {
-      const int k = q * 64 + lane, row = k / T::RC, c4 = k - row * T::RC;
-      const int m = m0 + T::WM * wm + 32 * half + row, n = n0 + T::WNC * wn + 4 * c4;
-      if (m >= P || n >= cout) continue;
-      const int at = m * cout + n;
-      const f32x4 o = *(const f32x4*)(stg + row * T::LS + 4 * c4);
-      if constexpr (OUT == VAE_RMS) {
-      } else if constexpr (OUT == VAE_BF16) {
-        *(u32x2*)((uint16_t*)Y + at) = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
-      } else if constexpr (OUT == VAE_PART) {
-        *(f32x4*)((float*)Y + (int64_t)z * P * cout + at) = o;
-      } else if constexpr (OUT == VAE_CLAMP) {
-        f32x4 c;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) c[e] = fminf(1.f, fmaxf(-1.f, o[e]));
-        *(f32x4*)((float*)Y + at) = c;
-      } else {
-        if (OUT != VAE_DUPUP || Y) *(f32x4*)((float*)Y + at) = o;   // DupUp: no fp32 out when Y is null
-        if constexpr (OUT == VAE_F32 || OUT == VAE_DUPUP) {
-          if (ep.y2) *(u32x2*)(ep.y2 + at) = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
-        }
-      }
-    }
-    if constexpr (GAM) {
-      static_assert(T::WNC == 144 || T::WNC == 96, "the norm's layout: rows of 144 or 96 a wave");
-      // each staged row's sum of squares: lanes 2r and 2r + 1 take its two halves, then swap; at
-      // BN 288 and 192 the row's other channels are the partner wave's (same pixels)
-      constexpr int HALF4 = T::WNC / 8;   // 4-channel chunks in half a row
-      const int rr = lane >> 1, hh = lane & 1;
-      float ss = 0.f;
-#pragma unroll 3
-      for (int c = 0; c < HALF4; ++c) {
-        const f32x4 t = *(const f32x4*)(stg + rr * T::LS + (T::WNC / 2) * hh + 4 * c);
-        ss += (t[0] * t[0] + t[1] * t[1]) + (t[2] * t[2] + t[3] * t[3]);
-      }
-      ss += dpp_f<0xB1>(ss);   // quad_perm [1, 0, 3, 2]: lane ^ 1
-      if constexpr (T::NWN == 2) {
-        if (hh == 0) stg[rr * T::LS + T::WNC] = ss;
-        __syncthreads();
-        const int partner = wn ? wave - T::NWM : wave + T::NWM;
-        ss += ((const float*)smem + partner * (32 * T::LS))[rr * T::LS + T::WNC];
-      }
-      const float inv = sqrtf((float)cout) / fmaxf(sqrtf(ss), 1e-12f);
-      if (hh == 0) stg[rr * T::LS + T::WNC + 1] = inv;
-      asm volatile("" ::: "memory");
-#pragma unroll 2
-      for (int q = 0; q < T::NCH; ++q) {
-        const int k = q * 64 + lane, row = k / T::RC, c4 = k - row * T::RC;
-        const int m = m0 + T::WM * wm + 32 * half + row, n = n0 + T::WNC * wn + 4 * c4;
-        if (m >= P) continue;
-        const f32x4 o = *(const f32x4*)(stg + row * T::LS + 4 * c4), g = *(const f32x4*)(ep.gamma + n);
-        const float iv = stg[row * T::LS + T::WNC + 1];
-        float e[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) e[j] = silu_bf16out(o[j] * iv * g[j]);
-        *(u32x2*)(ep.yr + (int64_t)m * cout + n) = u32x2{pack_bf16x2(e[0], e[1]), pack_bf16x2(e[2], e[3])};
-      }
-    }
+  for (int i = 0; i < NA_DMA; ++i) {
+    const int q = 64 * (T::NW * i + wave) + lane;
+    const int px = q >> 2, hy = px / HW, hx = px - hy * HW;
+    const int sy = (UP ? ty0 >> 1 : ty0) - 1 + hy, sx = (UP ? tx0 >> 1 : tx0) - 1 + hx;
+    const int c8 = (q & 3) ^ ((px >> 2) & 3);
+    aoff[i] = q < CHUNKS && sy >= 0 && sy < Hs && sx >= 0 && sx < Ws ? (uint32_t)(((sy * Ws + sx) * C + 8 * c8) * 2 + c8) : VOFF_NONE;
   }
+  auto a_dma = [&](int ch, int i) {   // round i of chunk ch's neighbourhood
+    uint8_t* st = smem + (ch & 1) * T::ABYTES;
+    uint32_t off = aoff[i];
+    asm volatile("" : "+v"(off));   // as in rd_a
+    off = 32 * ch + 8 * (int)(off & 3) < C ? off & ~3u : VOFF_NONE;
+    conv_dma(X, xext, (lds_void*)(st + (T::NW * i + wave) * 1024), off, ch * 64);
+  };
+  uint32_t boff[T::NB_DMA];
+#pragma unroll
+  for (int i = 0; i < T::NB_DMA; ++i) {
+    const int q = i < T::BFULL ? 64 * (T::NW * i + wave) + lane : 64 * T::NW * T::BFULL + T::BREM * wave + lane % (T::BREM ? T::BREM : 1);
+    const int row = q >> 2;
+    boff[i] = (uint32_t)((row * Kp + 8 * ((q & 3) ^ ((row >> 2) & 3))) * 2);
+  }
+  // round i of the weights of chunk ch's tap, k = tap C + 32 ch on
+  auto b_dma = [&](int ch, int tap, int s, int i) {
+    uint8_t* st = smem + 2 * T::ABYTES + s * T::BBYTES;
+    const int soff = (tap * C + 32 * ch) * 2;
+    if (i < T::BFULL) conv_dma(wbase, wext, (lds_void*)(st + (T::NW * i + wave) * 1024), boff[i], soff);
+    else if (lane < T::BREM) conv_dma(wbase, wext, (lds_void*)(st + T::NW * T::BFULL * 1024 + wave * T::BREM * 16), boff[i], soff);
+  };
+  // the fragments: row 4 wm + i of the tile at tap (q - 1, r - 1) is neighbourhood row 4 wm + i + q,
+  // column lo + r (UP: half of each, rounded down, one further)
+  const int pb = UP ? 2 * wm * HW : 4 * wm * HW + lo;
+  f32x4 acc[T::MI][T::NJ];
+#pragma unroll
+  for (int i = 0; i < T::MI; ++i)
+#pragma unroll
+    for (int j = 0; j < T::NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // the channel blocks in four groups, GO[g] .. GO[g + 1] - 1: two register sets serve them in turn
+  constexpr int GO[5] = {0, T::NJ == 9 ? 3 : 2, T::NJ == 9 ? 5 : 3, T::NJ == 9 ? 7 : 5, T::NJ};
+  bf16x8 fa[T::MI], fb[2][3];
+  auto rd_a = [&](int ch, int q, int r, int i) {   // q uniform; r and i known
+    int v = UP ? lo + r + 1 : pb;
+    asm volatile("" : "+v"(v));   // the addresses made anew each time: kept for every tap they spill
+    v = UP ? pb + HW * ((i + q + 1) >> 1) + (v >> 1) : v + HW * (i + q) + r;
+    fa[i] = *(const bf16x8*)(smem + (ch & 1) * T::ABYTES + v * 64 + ((q4 ^ ((v >> 2) & 3)) << 4));
+  };
+  const uint8_t* b_rd = smem + 2 * T::ABYTES + (T::WNC * wn + lo) * 64 + ((q4 ^ ((lo >> 2) & 3)) << 4);
+  auto rd_b = [&](int s, int j) { return *(const bf16x8*)(b_rd + s * T::BBYTES + j * 1024); };
+  auto landed = [&](auto keep) {   // all but the newest KEEP steps' weights, and every LDS read, for every wave
+    constexpr int VM = decltype(keep)::value * T::NB_DMA;
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((VM & 15) | (0x7 << 4) | (0x0 << 8) | ((VM >> 4) << 14));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+#pragma unroll
+  for (int i = 0; i < NA_DMA; ++i) a_dma(c0, i);
+#pragma unroll
+  for (int p = 0; p < T::NST; ++p)
+#pragma unroll
+    for (int i = 0; i < T::NB_DMA; ++i) b_dma(c0, p, p, i);
+  landed(std::integral_constant<int, T::NST - 1>());
+#pragma unroll
+  for (int j = 0; j < GO[1]; ++j) fb[0][j] = rd_b(0, j);
+#pragma unroll
+  for (int i = 0; i < T::MI; ++i) rd_a(c0, 0, 0, i);
+  int cur = 0;
+  for (int ch = c0; ch < c1; ++ch) {
+    // past the end the weights' DMA reloads the last chunk's, the neighbourhood's channels past C
+    // read as zeros, and nothing reads either
+    const int chn = min(ch + 1, c1 - 1);
+#pragma unroll 1
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+      for (int r = 0; r < 3; ++r) {
+        const int nx = cur + 1 == T::NST ? 0 : cur + 1;
+        // the next step's tap and chunk, and those of the step whose weights go out
+        const int qn = r < 2 ? q : q == 2 ? 0 : q + 1, cn = r == 2 && q == 2 ? ch + 1 : ch;
+        const int far = 3 * q + r + T::NST, fch = far < 9 ? ch : chn, ftap = far < 9 ? far : far - 9;
+#pragma unroll
+        for (int gr = 0; gr < 3; ++gr) {
+#pragma unroll
+          for (int j = GO[gr + 1]; j < GO[gr + 2]; ++j) fb[(gr + 1) & 1][j - GO[gr + 1]] = rd_b(cur, j);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < T::MI; ++i)
+#pragma unroll
+            for (int j = GO[gr]; j < GO[gr + 1]; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[gr & 1][j - GO[gr]], acc[i][j], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        // a wave's DMA lands in order, so that with the next step's weights everything older is
+        // in: the next chunk's neighbourhood, which goes out in the chunk's first three steps
+        landed(std::integral_constant<int, T::NST - 2>());
+#pragma unroll
+        for (int j = 0; j < GO[1]; ++j) fb[0][j] = rd_b(nx, j);
+        if (q == 0) {
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            if (2 * r + i < NA_DMA) a_dma(ch + 1, 2 * r + i);
+        }
+#pragma unroll
+        for (int i = 0; i < T::MI; ++i) {
+#pragma unroll
+          for (int j = GO[3]; j < GO[4]; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[1][j - GO[3]], acc[i][j], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          rd_a(cn, qn, r < 2 ? r + 1 : 0, i);
+          if (i < T::NB_DMA) b_dma(fch, ftap, cur, i);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        cur = nx;
+      }
+  }
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0x0 << 8));   // no DMA left in flight
+  asm volatile("" ::: "memory");
+  conv_epilogue<T, BN, OUT, GAM>(acc, smem, bias, ep, Y, P, W, cout, n0, wave, lane, wn, z, [&](int half, int row) {
+    const int y = ty0 + 4 * wm + 2 * half + (row >> 4), x = tx0 + (row & 15);
+    return y < H && x < W ? y * W + x : P;
+  });
 }
 
 // y = the S partial sums of a split-K convolution in order, + bias, + res when given; fp32 or
@@ -378,12 +571,35 @@ static hipError_t launch_conv1(hipStream_t s, const uint16_t* x, const uint16_t*
   return hipGetLastError();
 }
 
+// The 3 x 3 convolutions whose pictures 16 x 16 tiles cover with at most half as much again of
+// pixels off them (the linear tiles' step takes about 1.5 times as long), and whose weight rows
+// hold the last tap's last chunk (rows of 9 C rounded up to 64 do)
+static int64_t halo_tiles(int h, int w) { return (int64_t)((h + 15) / 16) * ((w + 15) / 16); }
+static bool halo_fits(int up, int h, int w, int c, int kp) {
+  return c >= 64 && halo_tiles(h, w) * 256 * 2 <= (int64_t)h * w * 3 && (!up || (h % 2 == 0 && w % 2 == 0)) &&
+         kp >= 8 * c + (c + 31) / 32 * 32;
+}
+
+template <int BN, int UP, int OUT, int GAM>
+static hipError_t launch_halo(hipStream_t s, const uint16_t* x, const uint16_t* wt, const float* bias, const VaeEpi& ep,
+                              void* y, int h, int w, int c, int cout, int kp, int split) {
+  auto kern = k_conv_halo<BN, UP, OUT, GAM>;
+  typedef HaloTile<BN> T;
+  const hipError_t e = ensure_lds((const void*)kern, T::LDS);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3((unsigned)halo_tiles(h, w), grid_of(cout, BN), split), dim3(T::NW * 64), T::LDS, s, x, wt,
+                     bias, ep, y, h, w, c, cout, kp);
+  return hipGetLastError();
+}
+
 // 128-pixel tiles of 4 waves (two workgroups a CU) for the 96- and 144-wide convolutions of
 // pictures of 2^18 pixels or more, where the output, residual and normed copy move as many bytes
 // as the products take time; 256-pixel tiles otherwise
 template <int BN, int TAPS, int UP, int OUT, int GAM = 0>
 static hipError_t launch_conv(hipStream_t s, const uint16_t* x, const uint16_t* wt, const float* bias, const VaeEpi& ep,
                               void* y, int h, int w, int c, int cout, int kp, int split = 1) {
+  if constexpr (TAPS == 9 && UP < 2 && BN > 16)
+    if (halo_fits(UP, h, w, c, kp)) return launch_halo<BN, UP, OUT, GAM>(s, x, wt, bias, ep, y, h, w, c, cout, kp, split);
   if constexpr (BN == 96 || BN == 144) {
     if (split == 1 && !ep.wide_only && (int64_t)h * w >= (1 << 18))
       return launch_conv1<BN, TAPS, UP, OUT, GAM, 4>(s, x, wt, bias, ep, y, h, w, c, cout, kp, 1);

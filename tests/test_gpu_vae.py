@@ -127,6 +127,26 @@ def test_conv_against_float64(ctx, case, split):
         assert np.abs(got - want).max() < 1e-4 * max(1.0, np.abs(want).max())
 
 
+HALO_CASES = [  # pictures that 16 x 16 tiles fit: whole tiles, edges one short and one past, odd sizes
+    ((16, 16, 64, 96, 9, 0, 0, True), False),
+    ((15, 31, 144, 144, 9, 0, 0, False), False),   # C = 4.5 chunks of 32: the last one's upper half zeros
+    ((47, 30, 288, 288, 9, 0, 1, True), False),
+    ((29, 45, 80, 192, 9, 0, 0, False), False),    # C no multiple of 32
+    ((32, 48, 576, 300, 9, 0, 2, False), False),   # output columns past whole tiles
+    ((32, 28, 288, 288, 9, 1, 0, False), False),   # the half-size picture's neighbourhoods, an edge inside a tile
+    ((14, 64, 144, 144, 9, 1, 0, False), False),
+    ((16, 32, 1152, 1152, 9, 0, 0, True), True),   # chunks split over workgroups
+    ((31, 16, 768, 768, 9, 0, 1, False), True),
+]
+
+
+@pytest.mark.parametrize("case,split", HALO_CASES)
+def test_conv_of_whole_neighbourhoods(ctx, case, split):
+    """As test_conv_against_float64, in the kernel that loads a tile's 18 x 18 (upsampling: 10 x 10)
+    neighbourhood once for the nine taps."""
+    test_conv_against_float64(ctx, case, split)
+
+
 def test_conv_rejects_bad_shapes(ctx):
     with pytest.raises(X.ExnError) as e:
         X.call("exn_vae_conv", ctx.h, 9, 0, 0, dev(ctx, np.zeros(64, np.uint16)).h, dev(ctx, np.zeros(64, np.uint16)).h,
