@@ -139,29 +139,34 @@ hipError_t rms_norm(hipStream_t s, int n, int width, float eps, const float* x, 
 // it), then each finished row's RMS norm times W into bf16 Y (4096 wide): the split sum's and
 // rms_norm's arithmetic in one pass over the rows.  One block a row; thread t takes columns
 // 4t + 1024j in both passes, as both separate kernels do, so the values are theirs bit for bit.
-// The row's 4 S partial loads go out before any sum.
-template <int S>
-__global__ void __launch_bounds__(256)
+// The row's 4 S partial loads go out before any sum.  WIDE: 1024 threads a row, a thread one of the
+// four column groups of thread t % 256 above (their squares added in the same order through LDS):
+// up to 512 rows leave a CU at most two of the 256-thread blocks, and a thread's 16 tanh and 4 S
+// loads are then the kernel's time (an encoder of 4 blocks, 8 of these: 378 -> 364 us at 24 rows,
+// 756 -> 739 at 256).
+template <int S, bool WIDE>
+__global__ void __launch_bounds__(WIDE ? 1024 : 256)
 k_sum_rms(int64_t M, const float* __restrict__ part, float* __restrict__ x, int64_t ldx, const float* __restrict__ gate,
           int n0, int p, int mstride, float eps, const float* __restrict__ w, uint16_t* __restrict__ y) {
   constexpr int64_t N = 4096;
-  __shared__ float red[4];
+  constexpr int J = WIDE ? 1 : 4;
+  __shared__ float red[4], sq[WIDE ? 1024 : 1];
   const int64_t m = blockIdx.x;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, c0 = 4 * (tid & 255) + 1024 * (tid >> 8);
   float* r = x + m * ldx;
   const float* gr = gate + (n0 + m < p ? mstride : 0);
-  f32x4 pv[4][S], xv[4];
+  f32x4 pv[J][S], xv[J];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int64_t c = 4 * tid + 1024 * j;
+  for (int j = 0; j < J; ++j) {
+    const int64_t c = c0 + 1024 * j;
 #pragma unroll
     for (int z = 0; z < S; ++z) pv[j][z] = *(const f32x4*)(part + ((int64_t)z * M + m) * N + c);
     xv[j] = *(const f32x4*)(r + c);
   }
   float ss = 0.f;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int64_t c = 4 * tid + 1024 * j;
+  for (int j = 0; j < J; ++j) {
+    const int64_t c = c0 + 1024 * j;
     f32x4 v = pv[j][0];
 #pragma unroll
     for (int z = 1; z < S; ++z) v += pv[j][z];
@@ -170,10 +175,22 @@ k_sum_rms(int64_t M, const float* __restrict__ part, float* __restrict__ x, int6
     *(f32x4*)(r + c) = xv[j];
     ss += xv[j][0] * xv[j][0] + xv[j][1] * xv[j][1] + xv[j][2] * xv[j][2] + xv[j][3] * xv[j][3];
   }
-  const float inv = rsqrtf(block_sum256(ss, red) / (float)N + eps);
+  if constexpr (WIDE) {
+    sq[tid] = ss;
+    __syncthreads();
+    if (tid < 256) {
+      ss = wave_sum_dpp(((sq[tid] + sq[tid + 256]) + sq[tid + 512]) + sq[tid + 768]);
+      if ((tid & 63) == 0) red[tid >> 6] = ss;
+    }
+    __syncthreads();
+    ss = red[0] + red[1] + red[2] + red[3];
+  } else {
+    ss = block_sum256(ss, red);
+  }
+  const float inv = rsqrtf(ss / (float)N + eps);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int64_t c = 4 * tid + 1024 * j;
+  for (int j = 0; j < J; ++j) {
+    const int64_t c = c0 + 1024 * j;
     const f32x4 wv = *(const f32x4*)(w + c);
     f32x4 o;
 #pragma unroll
@@ -187,11 +204,16 @@ hipError_t split_sum_rms(hipStream_t s, int S, int64_t M, int64_t N, const float
   if (M == 0) return hipSuccess;
   if (S < 1 || S > 8 || N != 4096 || ea.ldy % 4) return hipErrorInvalidValue;
   const dim3 g((unsigned)M);
+  const bool wide = M <= 512;
   switch (S) {
 #define EXN_SUM_RMS_S(k)                                                                                             \
   case k:                                                                                                            \
-    hipLaunchKernelGGL(k_sum_rms<k>, g, dim3(256), 0, s, M, part, ea.resid, ea.ldy, ea.gate, ea.n0, ea.p, ea.mstride, \
-                       eps, w, y);                                                                                   \
+    if (wide)                                                                                                        \
+      hipLaunchKernelGGL((k_sum_rms<k, true>), g, dim3(1024), 0, s, M, part, ea.resid, ea.ldy, ea.gate, ea.n0, ea.p, \
+                         ea.mstride, eps, w, y);                                                                     \
+    else                                                                                                             \
+      hipLaunchKernelGGL((k_sum_rms<k, false>), g, dim3(256), 0, s, M, part, ea.resid, ea.ldy, ea.gate, ea.n0, ea.p, \
+                         ea.mstride, eps, w, y);                                                                     \
     break;
     EXN_SUM_RMS_S(1) EXN_SUM_RMS_S(2) EXN_SUM_RMS_S(3) EXN_SUM_RMS_S(4) EXN_SUM_RMS_S(5) EXN_SUM_RMS_S(6)
     EXN_SUM_RMS_S(7) EXN_SUM_RMS_S(8)
