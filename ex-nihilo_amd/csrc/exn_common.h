@@ -303,7 +303,7 @@ struct VaeEpi {
   // head's normed input; VAE_RMS writes yr only
   const float* gamma;
   uint16_t* yr;
-  // 1: 256-pixel tiles always (the 128-pixel ones of large pictures off; the same sums, a test's
+  // 1: k_conv's 256-pixel tiles always (its 128-pixel ones of large pictures off; the same sums, a test's
   // switch)
   int wide_only;
 };
