@@ -1357,7 +1357,8 @@ static bool few_fits(const uint16_t* x, int64_t lda, const WOp& w, int64_t M, in
 // Every load is a buffer load whose vector offset the extent covers: rows past M and steps past
 // the wave's last read as zeros.  At 24 rows gate_up (107 MB of codes and scales) took 36.2 us and
 // a split sum of 4.6 there, 28.9 here (3.7 TB/s); to_out and down 20.5 on average, 14.6 here; an
-// encoder of 4 blocks 474 -> 376 us (8 rows 454 -> 328, 48 rows 496 -> 456, 64 rows 509 -> 508).
+// encoder of 4 blocks 474 -> 376 us (8 rows 454 -> 328, 48 rows 496 -> 456), with rows_split 338
+// (291, 422).
 template <int EPI, int MI, bool Q8>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_gemm_rows(const uint16_t* __restrict__ X, int64_t lda, const uint16_t* __restrict__ WB,
@@ -1508,11 +1509,13 @@ k_gemm_rows(const uint16_t* __restrict__ X, int64_t lda, const uint16_t* __restr
 
 #define ROWS_MAX 48   // at 64 rows (4 row fragments) X's stream from L2 passes W's and nothing is won
 
-// how many workgroups a tile's K is split over: about 1.5 workgroups a CU, each wave at least two
-// steps, at most SMAX
-static int64_t rows_split(int64_t N, int64_t K, int64_t smax) {
+// how many workgroups a tile's K is split over: 192 workgroups in all, each wave at least two
+// steps, at most SMAX; 256 past 32 rows, where a wave holds two steps and not four.  An encoder of 4
+// blocks at 24 and 48 rows (us): 96 workgroups 372 and 501, 160 338 and 428, 192 338 and 428, 256
+// 346 and 422, 384 364 and 443, 512 386 and 437: fewer leave CUs idle, more pay for partial sums.
+static int64_t rows_split(int64_t M, int64_t N, int64_t K, int64_t smax) {
   const int64_t tiles = N / 64;
-  int64_t S = (384 + tiles - 1) / tiles;
+  int64_t S = ((M <= 32 ? 192 : 256) + tiles - 1) / tiles;
   if (S > K / 64 / 8) S = K / 64 / 8;
   if (S > smax) S = smax;
   return S < 1 ? 1 : S;
@@ -1666,7 +1669,7 @@ hipError_t gemm_split_rows(hipStream_t s, const uint16_t* x, int64_t lda, const 
     // at most 256 rows: the few-row tiles, K split so that the tiles' workgroups are about one a
     // CU, each at least 4 k-steps, at most SMAX ways and within PART_CAP
     const int64_t tiles = N / (M > 128 ? 128 : 256);
-    int64_t S = M <= ROWS_MAX ? rows_split(N, K, smax) : 256 / tiles;
+    int64_t S = M <= ROWS_MAX ? rows_split(M, N, K, smax) : 256 / tiles;
     if (S > K / 256) S = K / 256;
     if (S > smax) S = smax;
     if (S > part_cap / (M * N)) S = part_cap / (M * N);
