@@ -490,6 +490,20 @@ int exn_mm_w8a8(exn_ctx* ctx, const exn_w* w, const int8_t* xq, const uint16_t* 
   return EXN_OK;
 }
 
+int exn_mm_w8a8_swiglu(exn_ctx* ctx, const exn_w* w, const int8_t* xq, const uint16_t* xd, int64_t n, int8_t* q,
+                       uint16_t* d) {
+  TRY(use(ctx));
+  if (!w || w->kind != EXN_Q8_0 || w->dense || !w->qs) FAIL(EXN_EINVAL, "mm_w8a8_swiglu: the matrix is not Q8_0");
+  if (!w->pairs) FAIL(EXN_EINVAL, "exn_mm_w8a8_swiglu wants a matrix interleaved by exn_weight_pairs");
+  if (!xq || !xd || !q || !d || n < 0) FAIL(EXN_EINVAL, "mm_w8a8_swiglu arguments");
+  const hipError_t e = gemm_w8a8_swiglu(ctx->stream, xq, xd, n, w->qs, w->d, w->rows, w->cols, q, d);
+  if (e == hipErrorNotSupported)
+    FAIL(EXN_EINVAL, "mm_w8a8_swiglu: %lld x %lld over %lld rows (multiples of 64, 16-byte aligned arrays)",
+         (long long)w->rows, (long long)w->cols, (long long)n);
+  HIPCHK(e);
+  return EXN_OK;
+}
+
 int exn_euler(exn_ctx* ctx, int64_t count, float* z, const float* v, float ds) {
   TRY(use(ctx));
   if (count < 0 || !z || !v) FAIL(EXN_EINVAL, "euler arguments");

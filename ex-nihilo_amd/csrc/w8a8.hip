@@ -361,6 +361,7 @@ k_gemm_w8a8_dma(const int8_t* __restrict__ xq, const uint16_t* __restrict__ xd, 
     __syncthreads();
     int8_t* codes = (int8_t*)smem + wave * 2048;
     const int64_t blk = (tn + wn) >> 6, KBO = N >> 6;
+    if (tn + wn >= N) return;   // the last tile's right waves at N % 128 == 64: no block of theirs
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll

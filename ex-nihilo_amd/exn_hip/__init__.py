@@ -68,6 +68,7 @@ SIGNATURES = {
     "exn_mm_noalloc": (c_int, [vp, vp, vp, c_int, vp, c_int, c_int64]),
     "exn_quant_q8": (c_int, [vp, vp, c_int, c_int64, c_int64, c_int64, vp, vp]),
     "exn_mm_w8a8": (c_int, [vp, vp, vp, vp, c_int64, vp, c_int]),
+    "exn_mm_w8a8_swiglu": (c_int, [vp, vp, vp, vp, c_int64, vp, vp]),
     "exn_mm_gate_add": (c_int, [vp, vp, vp, c_int64, vp, c_int, c_int, c_int, vp]),
     "exn_mm_swiglu": (c_int, [vp, vp, vp, vp, c_int64]),
     "exn_weight_pairs": (c_int, [vp, vp]),

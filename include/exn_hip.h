@@ -121,6 +121,11 @@ int exn_quant_q8(exn_ctx* ctx, const void* x, int xdt, int64_t ldx, int64_t n, i
  * y = fma(float(isum), dx * dw, y) in fp32 over the blocks in order; Y [n][rows] fp32 or fp16
  * (EXN_DT_F32 / EXN_DT_F16) */
 int exn_mm_w8a8(exn_ctx* ctx, const exn_w* w, const int8_t* xq, const uint16_t* xd, int64_t n, void* y, int ydt);
+/* exn_mm_w8a8 of a paired gate_up matrix (exn_weight_pairs; rows and cols multiples of 64), then
+ * SwiGLU and exn_quant_q8 of its rows fused into the product's store: Q int8 [n][rows / 2], D fp16
+ * [n][rows / 64], the values of the steps apart bit for bit */
+int exn_mm_w8a8_swiglu(exn_ctx* ctx, const exn_w* w, const int8_t* xq, const uint16_t* xd, int64_t n, int8_t* q,
+                       uint16_t* d);
 /* mm, then x_gate_add fused into the product's store (src/cuda/dit.cu:34-41):
  * RESID[t] += tanh(GATE[row]) * (X W^T)[t]; sequence row N0 + t < P takes GATE + MSTRIDE */
 int exn_mm_gate_add(exn_ctx* ctx, const exn_w* w, const uint16_t* x_bf16, int64_t n, float* resid, int n0, int p,

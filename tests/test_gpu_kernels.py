@@ -657,6 +657,34 @@ def test_mm_w8a8_bit_exact(ctx, M, N, K):
     assert np.array_equal(y16.get(), want.astype(np.float16).view(np.uint16))
 
 
+@pytest.mark.parametrize("M,N", [(1, 64), (70, 192), (128, 256), (130, 320), (129, 192)])
+def test_mm_w8a8_swiglu_stores_its_own_blocks_only(ctx, M, N):
+    """exn_mm_w8a8_swiglu against exn_mm_w8a8 of the same matrix before its interleave, SwiGLU and
+    quant_q8_0 on the host, at widths that end on half a 128-column tile (N % 128 == 64), on ragged
+    rows: the bytes behind both outputs stay as they were, and every row's blocks are its own.  The
+    host's exp is not the device's, each within 2 ulp, so a value is within 2^-20: a code may fall
+    on the other side of a half (one apart, one in 100 at most), a scale on that of an fp16 tie."""
+    say("mm_w8a8_swiglu", M, N)
+    K, F = 256, N // 2
+    x = np.random.default_rng(M + N).normal(0, 2, (M, K)).astype(np.float32)
+    q, dd = X.DevBuf(ctx, (M, K), np.int8), X.DevBuf(ctx, (M, K // 32), np.uint16)
+    X.call("exn_quant_q8", ctx.h, dev(ctx, x).h, X.DT_F32, K, M, K, q.h, dd.h)
+    y = X.DevBuf(ctx, (M, N), np.float32)
+    w = X.Weight.synth(ctx, 14, 500 + N, N, K)
+    X.call("exn_mm_w8a8", ctx.h, w.h, q.h, dd.h, M, y.h, X.DT_F32)
+    gu = y.get().astype(np.float64)
+    want = (gu[:, :F] / (1 + np.exp(-gu[:, :F])) * gu[:, F:]).astype(np.float32)
+    wq, wd = xo.quant_q8_0(want)
+    w.pairs()
+    oq, od = dev(ctx, np.full(M * F + 4096, 77, np.int8)), dev(ctx, np.full(M * F // 32 + 128, 0x7777, np.uint16))
+    X.call("exn_mm_w8a8_swiglu", ctx.h, w.h, q.h, dd.h, M, oq.h, od.h)
+    gq, gd = oq.get(), od.get()
+    assert (gq[M * F:] == 77).all() and (gd[M * F // 32:] == 0x7777).all()
+    off = np.abs(gq[:M * F].reshape(M, F).astype(int) - wq)
+    assert off.max() <= 1 and off.sum() <= max(1, M * F // 100)
+    assert np.abs(gd[:M * F // 32].reshape(M, -1).astype(int) - wd.view(np.uint16)).max() <= 1
+
+
 def test_allocation_failure_is_a_status(ctx):
     """exn_alloc of an absurd size (1 PiB) returns EXN_ENOMEM with a message naming the size,
     raises nothing, and leaves the context usable: a buffer, an upload and a product after it."""
