@@ -674,6 +674,13 @@ int exn_vae_conv(exn_ctx* ctx, int taps, int up, int outdt, const uint16_t* x, c
   return EXN_OK;
 }
 
+int exn_vae_conv_way(int up, int h, int w, int c, int cout, int64_t part_cap, int* square, int* split, int64_t* groups) {
+  if (!square || !split || !groups || up < 0 || up > 1 || h <= 0 || w <= 0 || c < 64 || c % 8 || cout <= 16 || cout % 4 || part_cap < 0)
+    FAIL(EXN_EINVAL, "vae conv way arguments");
+  vae_conv_way(up, h, w, c, cout, (9 * c + 63) / 64 * 64, up ? 0 : part_cap, square, split, groups);
+  return EXN_OK;
+}
+
 int exn_vae_rms_silu(exn_ctx* ctx, int64_t n, int c, const float* x, const float* gamma, uint16_t* y, int silu) {
   TRY(use(ctx));
   if (!x || !gamma || !y || c % 4 || n < 0) FAIL(EXN_EINVAL, "vae rms arguments");

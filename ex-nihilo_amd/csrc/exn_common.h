@@ -307,6 +307,9 @@ struct VaeEpi {
   // switch)
   int wide_only;
 };
+// the tiles (SQUARE: k_conv_halo's), K split and workgroups of a 3 x 3 convolution with PARTS floats of
+// split-K scratch
+void vae_conv_way(int up, int h, int w, int c, int cout, int kp, int64_t parts, int* square, int* split, int64_t* groups);
 hipError_t vae_conv(hipStream_t s, int taps, int up, int out, const uint16_t* x, const uint16_t* wt,
                     const float* bias, const VaeEpi& ep, void* y, int h, int w, int c, int cout, int kp);
 hipError_t vae_rms_silu(hipStream_t s, int64_t P, int C, const float* x, const float* gamma, uint16_t* y, int silu);

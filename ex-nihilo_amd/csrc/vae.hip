@@ -26,6 +26,7 @@
 // so that bias, residual, DupUp3D and clamp are applied to 16-byte rows.
 #include "exn_common.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace exn {
@@ -571,13 +572,43 @@ static hipError_t launch_conv1(hipStream_t s, const uint16_t* x, const uint16_t*
   return hipGetLastError();
 }
 
-// The 3 x 3 convolutions whose pictures 16 x 16 tiles cover with at most half as much again of
-// pixels off them (the linear tiles' step takes about 1.5 times as long), and whose weight rows
-// hold the last tap's last chunk (rows of 9 C rounded up to 64 do)
+// k_conv_halo takes pictures that 16 x 16 tiles cover with at most half as much again of pixels off
+// them, whose weight rows hold the last tap's last chunk (rows of 9 C rounded up to 64 do)
 static int64_t halo_tiles(int h, int w) { return (int64_t)((h + 15) / 16) * ((w + 15) / 16); }
 static bool halo_fits(int up, int h, int w, int c, int kp) {
   return c >= 64 && halo_tiles(h, w) * 256 * 2 <= (int64_t)h * w * 3 && (!up || (h % 2 == 0 && w % 2 == 0)) &&
          kp >= 8 * c + (c + 31) / 32 * 32;
+}
+
+// How a 3 x 3 convolution runs: its kernel, and how many workgroups share a tile's K
+struct ConvWay {
+  bool halo;
+  int split;
+};
+
+// A convolution of fewer tiles than the chip's CUs (the decoder's 64 x 64 stages: 64 tiles) splits
+// its K over up to 4 workgroups a tile, each at least 16 k-steps, where PARTS has room (floats; 0:
+// none); k_part_sum adds them in order.  Each kernel's split follows its own grid: 36 x 128 pixels of
+// 1152 channels are 72 linear tiles, 3 ways, but 96 square ones, 2 ways.
+static int conv_split(int64_t tiles, int64_t out, int kp, int64_t parts) {
+  int64_t s = std::min<int64_t>(std::min<int64_t>(256 / tiles, 4), kp / 64 / 16);
+  if (tiles >= 192 || s < 2 || s * out > parts) s = 1;
+  return (int)s;
+}
+
+// The neighbourhood kernel where its waves of workgroups, each a split's share of K long, cost no more
+// than the linear tiles', whose steps take at least 1.1 times as long (the kernel's table: 1.10 to
+// 1.38).  36 x 128 x 1152 -> 1152: 120 us on linear tiles 3 ways, 187 on square ones split as many
+// ways, which are two waves.
+template <int BN>
+static ConvWay conv_way(int up, int h, int w, int c, int cout, int kp, int64_t parts) {
+  const int64_t P = (int64_t)h * w, gn = grid_of(cout, BN);
+  const int64_t lt = grid_of(P, ConvTile<BN>::TM) * gn, ht = halo_tiles(h, w) * gn;
+  const ConvWay lin{false, conv_split(lt, P * cout, kp, parts)}, halo{true, conv_split(ht, P * cout, kp, parts)};
+  if (!halo_fits(up, h, w, c, kp)) return lin;
+  const double cl = 1.1 * (double)((lt * lin.split + 255) / 256) / lin.split;
+  const double ch = (double)((ht * halo.split + 255) / 256) / halo.split;
+  return ch <= cl ? halo : lin;
 }
 
 template <int BN, int UP, int OUT, int GAM>
@@ -597,9 +628,10 @@ static hipError_t launch_halo(hipStream_t s, const uint16_t* x, const uint16_t* 
 // as the products take time; 256-pixel tiles otherwise
 template <int BN, int TAPS, int UP, int OUT, int GAM = 0>
 static hipError_t launch_conv(hipStream_t s, const uint16_t* x, const uint16_t* wt, const float* bias, const VaeEpi& ep,
-                              void* y, int h, int w, int c, int cout, int kp, int split = 1) {
+                              void* y, int h, int w, int c, int cout, int kp, ConvWay way = {false, 1}) {
+  const int split = way.split;
   if constexpr (TAPS == 9 && UP < 2 && BN > 16)
-    if (halo_fits(UP, h, w, c, kp)) return launch_halo<BN, UP, OUT, GAM>(s, x, wt, bias, ep, y, h, w, c, cout, kp, split);
+    if (way.halo) return launch_halo<BN, UP, OUT, GAM>(s, x, wt, bias, ep, y, h, w, c, cout, kp, split);
   if constexpr (BN == 96 || BN == 144) {
     if (split == 1 && !ep.wide_only && (int64_t)h * w >= (1 << 18))
       return launch_conv1<BN, TAPS, UP, OUT, GAM, 4>(s, x, wt, bias, ep, y, h, w, c, cout, kp, 1);
@@ -613,15 +645,14 @@ template <int BN>
 static hipError_t conv_bn(hipStream_t s, int taps, int up, int out, const uint16_t* x, const uint16_t* wt,
                           const float* bias, const VaeEpi& ep, void* y, int h, int w, int c, int cout, int kp) {
   constexpr bool DEC = ConvTile<BN>::WNC == 144;
-  // a 3 x 3 convolution of fewer tiles than the chip's CUs (the decoder's 64 x 64 stages: 64
-  // tiles) splits its K over up to 4 workgroups a tile, each at least 16 k-steps, into fp32
-  // partials; k_part_sum adds them in order with bias and res
+  const bool splits = taps == 9 && !up && (out == VAE_F32 || out == VAE_BF16) && !ep.y2 && ep.part && !ep.gamma;
+  const ConvWay way = taps == 9 && up < 2 ? conv_way<BN>(up, h, w, c, cout, kp, splits ? ep.part_cap : 0) : ConvWay{false, 1};
   if (ep.gamma) {   // the output's norm too: one channel tile (cout == BN), never split
-    if (taps == 9 && !up && out == VAE_F32) return launch_conv<BN, 9, 0, VAE_F32, 1>(s, x, wt, bias, ep, y, h, w, c, cout, kp);
-    if (taps == 9 && !up && out == VAE_RMS) return launch_conv<BN, 9, 0, VAE_RMS, 1>(s, x, wt, bias, ep, y, h, w, c, cout, kp);
+    if (taps == 9 && !up && out == VAE_F32) return launch_conv<BN, 9, 0, VAE_F32, 1>(s, x, wt, bias, ep, y, h, w, c, cout, kp, way);
+    if (taps == 9 && !up && out == VAE_RMS) return launch_conv<BN, 9, 0, VAE_RMS, 1>(s, x, wt, bias, ep, y, h, w, c, cout, kp, way);
     if constexpr (DEC) {
       if (taps == 9 && up == 1 && out == VAE_DUPUP)
-        return launch_conv<BN, 9, 1, VAE_DUPUP, 1>(s, x, wt, bias, ep, y, h, w, c, cout, kp);
+        return launch_conv<BN, 9, 1, VAE_DUPUP, 1>(s, x, wt, bias, ep, y, h, w, c, cout, kp, way);
     } else {
       // the encoder's first convolution (a 1 x 1 product over RGBA neighbourhoods) with the
       // first block's normed input
@@ -629,28 +660,43 @@ static hipError_t conv_bn(hipStream_t s, int taps, int up, int out, const uint16
     }
     return hipErrorInvalidValue;
   }
-  const int64_t P = (int64_t)h * w, tiles = grid_of(P, ConvTile<BN>::TM) * (int64_t)grid_of(cout, BN);
-  int64_t split = 256 / tiles < 4 ? 256 / tiles : 4;
-  if (kp / 64 / 16 < split) split = kp / 64 / 16;
-  if (taps == 9 && !up && (out == VAE_F32 || out == VAE_BF16) && !ep.y2 && ep.part && tiles < 192 && split >= 2 &&
-      split * P * cout <= ep.part_cap) {
-    hipError_t e = launch_conv<BN, 9, 0, VAE_PART>(s, x, wt, bias, ep, ep.part, h, w, c, cout, kp, (int)split);
+  if (splits && way.split > 1) {
+    hipError_t e = launch_conv<BN, 9, 0, VAE_PART>(s, x, wt, bias, ep, ep.part, h, w, c, cout, kp, way);
     if (e != hipSuccess) return e;
-    return part_sum(s, (int)split, P * cout, cout, ep.part, bias, ep.res, y, out == VAE_BF16);
+    return part_sum(s, way.split, (int64_t)h * w * cout, cout, ep.part, bias, ep.res, y, out == VAE_BF16);
   }
-  if (taps == 9 && !up && out == VAE_F32) return launch_conv<BN, 9, 0, VAE_F32>(s, x, wt, bias, ep, y, h, w, c, cout, kp);
-  if (taps == 9 && !up && out == VAE_BF16) return launch_conv<BN, 9, 0, VAE_BF16>(s, x, wt, bias, ep, y, h, w, c, cout, kp);
+  if (taps == 9 && !up && out == VAE_F32) return launch_conv<BN, 9, 0, VAE_F32>(s, x, wt, bias, ep, y, h, w, c, cout, kp, way);
+  if (taps == 9 && !up && out == VAE_BF16) return launch_conv<BN, 9, 0, VAE_BF16>(s, x, wt, bias, ep, y, h, w, c, cout, kp, way);
   if constexpr (DEC) {
-    if (taps == 9 && !up && out == VAE_CLAMP) return launch_conv<BN, 9, 0, VAE_CLAMP>(s, x, wt, bias, ep, y, h, w, c, cout, kp);
-    if (taps == 9 && up == 1 && out == VAE_F32) return launch_conv<BN, 9, 1, VAE_F32>(s, x, wt, bias, ep, y, h, w, c, cout, kp);
+    if (taps == 9 && !up && out == VAE_CLAMP) return launch_conv<BN, 9, 0, VAE_CLAMP>(s, x, wt, bias, ep, y, h, w, c, cout, kp, way);
+    if (taps == 9 && up == 1 && out == VAE_F32) return launch_conv<BN, 9, 1, VAE_F32>(s, x, wt, bias, ep, y, h, w, c, cout, kp, way);
     if (taps == 9 && up == 1 && out == VAE_DUPUP)
-      return launch_conv<BN, 9, 1, VAE_DUPUP>(s, x, wt, bias, ep, y, h, w, c, cout, kp);
+      return launch_conv<BN, 9, 1, VAE_DUPUP>(s, x, wt, bias, ep, y, h, w, c, cout, kp, way);
   } else {
     if (taps == 9 && up == 2 && out == VAE_F32) return launch_conv<BN, 9, 2, VAE_F32>(s, x, wt, bias, ep, y, h, w, c, cout, kp);
   }
   if (taps == 1 && !up && out == VAE_F32) return launch_conv<BN, 1, 0, VAE_F32>(s, x, wt, bias, ep, y, h, w, c, cout, kp);
   if (taps == 1 && !up && out == VAE_BF16) return launch_conv<BN, 1, 0, VAE_BF16>(s, x, wt, bias, ep, y, h, w, c, cout, kp);
   return hipErrorInvalidValue;
+}
+
+// the channel tile of a convolution: the wide one where 288 divides the width (1152, 576, 288 and the
+// 3456 of q|k|v); 192 and 96 for the encoder's widths (96, 192, 384, 768); else 144, the decoder's
+static int conv_tile(int cout) {
+  if (cout % 288 == 0) return 288;
+  if (cout % 144 != 0 && cout % 192 == 0) return 192;
+  return cout % 144 != 0 && cout % 96 == 0 ? 96 : 144;
+}
+
+void vae_conv_way(int up, int h, int w, int c, int cout, int kp, int64_t parts, int* square, int* split, int64_t* groups) {
+  const int bn = conv_tile(cout);
+  const ConvWay y = bn == 288   ? conv_way<288>(up, h, w, c, cout, kp, parts)
+                    : bn == 192 ? conv_way<192>(up, h, w, c, cout, kp, parts)
+                    : bn == 96  ? conv_way<96>(up, h, w, c, cout, kp, parts)
+                                : conv_way<144>(up, h, w, c, cout, kp, parts);
+  *square = y.halo;
+  *split = y.split;
+  *groups = (y.halo ? halo_tiles(h, w) : (int64_t)grid_of((int64_t)h * w, 256)) * grid_of(cout, bn) * y.split;
 }
 
 hipError_t vae_conv(hipStream_t s, int taps, int up, int out, const uint16_t* x, const uint16_t* wt, const float* bias,
@@ -671,12 +717,11 @@ hipError_t vae_conv(hipStream_t s, int taps, int up, int out, const uint16_t* x,
       (out == VAE_DUPUP && (!ep.keep || ep.ft < 1 || ep.kcin <= 0 || (int64_t)cout * ep.ft * 4 % ep.kcin || h % 2 ||
                             w % 2 || ((cout * ep.ft * 4 / ep.kcin) & (cout * ep.ft * 4 / ep.kcin - 1)))))
     return hipErrorInvalidValue;
-  // the wide tile where 288 divides the width (1152, 576, 288 and the 3456 of q|k|v); 144 for
-  // the decoder's 144; 192 and 96 for the encoder's widths (96, 192, 384, 768); a narrow one
-  // for a few channels (the head's 4): 16 columns of MFMA work instead of 144
-  if (cout % 288 == 0) return conv_bn<288>(s, taps, up, out, x, wt, bias, ep, y, h, w, c, cout, kp);
-  if (cout % 144 != 0 && cout % 192 == 0) return conv_bn<192>(s, taps, up, out, x, wt, bias, ep, y, h, w, c, cout, kp);
-  if (cout % 144 != 0 && cout % 96 == 0) return conv_bn<96>(s, taps, up, out, x, wt, bias, ep, y, h, w, c, cout, kp);
+  const int bn = conv_tile(cout);
+  if (bn == 288) return conv_bn<288>(s, taps, up, out, x, wt, bias, ep, y, h, w, c, cout, kp);
+  if (bn == 192) return conv_bn<192>(s, taps, up, out, x, wt, bias, ep, y, h, w, c, cout, kp);
+  if (bn == 96) return conv_bn<96>(s, taps, up, out, x, wt, bias, ep, y, h, w, c, cout, kp);
+  // a few channels (the head's 4): 16 columns of MFMA work instead of 144
   if (cout <= 16 && !ep.gamma) {
     if (taps == 9 && !up && out == VAE_CLAMP) return launch_conv<16, 9, 0, VAE_CLAMP>(s, x, wt, bias, ep, y, h, w, c, cout, kp);
     if (taps == 9 && !up && out == VAE_F32) return launch_conv<16, 9, 0, VAE_F32>(s, x, wt, bias, ep, y, h, w, c, cout, kp);

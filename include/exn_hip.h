@@ -316,6 +316,10 @@ int exn_vae_tiles(exn_vae* v, int small);
  * over up to 4 workgroups a tile and sums their partials in order. */
 int exn_vae_conv(exn_ctx* ctx, int taps, int up, int outdt, const uint16_t* x, const uint16_t* wt, const float* bias,
                  const float* res, void* y, int h, int w, int c, int cout, int kp, float* part, int64_t part_cap);
+/* test hook, needs no GPU: how a 3 x 3 convolution (UP 0 or 1) of an H x W output and PART_CAP floats
+ * of PART runs: SQUARE 1 on 16 x 16-pixel tiles whose neighbourhood is loaded once, 0 on runs of
+ * 256 pixels; SPLIT workgroups a tile's K is split over; GROUPS workgroups in all */
+int exn_vae_conv_way(int up, int h, int w, int c, int cout, int64_t part_cap, int* square, int* split, int64_t* groups);
 int exn_vae_rms_silu(exn_ctx* ctx, int64_t n, int c, const float* x, const float* gamma, uint16_t* y, int silu);
 int exn_vae_dupup_add(exn_ctx* ctx, int cin, int cout, int ft, int h, int w, const float* x, float* y);
 /* Y (H/2 x W/2 x COUT) += AvgDown3D(X) (H x W x CIN), frame FT - 1 of FT */

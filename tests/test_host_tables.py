@@ -3,6 +3,8 @@ positions every sequence row gets (dit-positions, src/host.lisp:37-50; integer
 work, bit-exact) and the cos/sin table the step uploads (rope-table,
 src/host.lisp:19-30; within one float32 ulp), through the C ABI test hook
 exn_dit_rope_table, for odd image sizes and for edit layouts with rh != rw."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -72,3 +74,37 @@ def test_encoder_rope_table_matches_the_oracle(case):
     cs = X.enc_rope_table(len(pos), None if case == "text" else pos)
     cos, sin = eo.mrope_tables(pos)
     assert ulps(cs[:, 0::2], cos).max() <= 1 and ulps(cs[:, 1::2], sin).max() <= 1
+
+
+# --- the VAE's convolutions: tiles and K split ----------------------------------------------
+
+def conv_way(up, h, w, c, cout, cap):
+    a, b, g = ctypes.c_int(), ctypes.c_int(), ctypes.c_int64()
+    X.call("exn_vae_conv_way", up, h, w, c, cout, cap, ctypes.byref(a), ctypes.byref(b), ctypes.byref(g))
+    return a.value, b.value, g.value
+
+
+def test_split_convolutions_stay_within_one_wave():
+    """A convolution's K is split to fill the 256 CUs once: no stage of any latent of 4 x 4 to
+    40 x 64 has a split whose workgroups pass 256 (a second wave, as long as the first), on either
+    kind of tiles, nor one past the scratch; without scratch none is split."""
+    ways = set()
+    for h in range(4, 41, 3):
+        for w in range(4, 65):
+            for s, c, cout in ((1, 1152, 1152), (2, 1152, 1152), (4, 1152, 1152), (4, 1152, 576), (1, 768, 768),
+                               (2, 768, 768), (4, 384, 384), (8, 192, 192), (1, 768, 128)):
+                H, W, cap = h * s, w * s, 4 << 24
+                square, split, groups = conv_way(0, H, W, c, cout, cap)
+                ways.add((square, split))
+                assert split == 1 or (groups <= 256 and split * H * W * cout <= cap), (H, W, c, cout, square, split)
+                assert conv_way(0, H, W, c, cout, 0)[1] == 1 and conv_way(1, 2 * H, 2 * W, c, cout, cap)[1] == 1
+    assert ways == {(a, b) for a in (0, 1) for b in (1, 2, 3, 4)}
+
+
+def test_convolutions_take_the_tiles_of_the_fewer_steps():
+    """36 x 128 pixels of 1152 channels: 72 runs of 256 pixels 3 ways before 96 squares 2 ways; 64 x 64:
+    64 of either 4 ways, the squares; a picture mostly off its squares: runs."""
+    assert conv_way(0, 36, 128, 1152, 1152, 1 << 26) == (0, 3, 216)
+    assert conv_way(0, 64, 64, 1152, 1152, 1 << 26) == (1, 4, 256)
+    assert conv_way(0, 1024, 1024, 144, 144, 0) == (1, 1, 4096)
+    assert conv_way(0, 17, 4, 1152, 1152, 1 << 26) == (0, 4, 16)
