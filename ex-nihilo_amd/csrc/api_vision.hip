@@ -57,9 +57,11 @@ std::vector<VExpect> vision_expected() {
 }  // namespace
 
 // what a split product needs of a weight: the largest |x|, the largest row's 2-norm (a vector is
-// one row) and, of a matrix whose values are fp16 times 2^-kw, those fp16 rows (kp apart)
+// one row) and, of a matrix whose values are fp16 times 2^-kw, those fp16 rows (kp apart).  Those of
+// a tensor stored and not (yet) measured bound nothing: its products, and those that its bounds
+// reach, run in fp32
 struct VisFacts {
-  double mx = 0, norm = 0;
+  double mx = INFINITY, norm = INFINITY;
   uint16_t* h = nullptr;
   int kp = 0, kw = 0;
   bool exact = false;
@@ -128,11 +130,14 @@ static const float* vis_t(const exn_vision* v, const std::string& name) {
 
 // N fp32 values (device, DATA) into tensor NAME's device copy
 static int vis_store(exn_vision* v, const std::string& name, int64_t n, const float* data) {
+  VisFacts& f = v->facts[name];   // the old values' go first: what follows may fail
+  f.mx = f.norm = INFINITY;
+  f.exact = false;
+  v->plan_ok = false;
   float*& p = v->t[name];
   if (!p) TRY(dev_alloc((void**)&p, (size_t)n * 4));
   HIPCHK(hipMemcpyAsync(p, data, (size_t)n * 4, hipMemcpyDeviceToDevice, v->ctx->stream));
   if (name.rfind("v.patch_embd.weight", 0) == 0) v->pw_ok = false;
-  v->plan_ok = false;
   return EXN_OK;
 }
 
