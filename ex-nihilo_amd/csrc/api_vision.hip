@@ -174,11 +174,12 @@ static int vis_measure(exn_vision* v, const std::vector<size_t>& which) {
     if (!used(which[j])) continue;
     const VExpect& e = v->expect[which[j]];
     VisFacts& f = v->facts[e.name];
-    float mx, ss;
+    float mx;
+    double ss;
     memcpy(&mx, &host[4 * j], 4);
-    memcpy(&ss, &host[4 * j + 1], 4);
+    memcpy(&ss, &host[4 * j + 2], 8);
     f.mx = mx;
-    f.norm = std::sqrt((double)ss) * 1.001;   // the sum's own rounding
+    f.norm = std::sqrt(ss) * 1.001;   // the sum's own rounding
     f.exact = false;
     if (e.shape.size() < 2 || !std::isfinite(mx)) continue;
     dims(which[j], rows, cols);
@@ -186,19 +187,20 @@ static int vis_measure(exn_vision* v, const std::vector<size_t>& which) {
     f.kw = mx > 0.f ? std::min(40, std::max(0, 14 - std::ilogb(mx))) : 0;
     if (!f.h && dev_alloc((void**)&f.h, (size_t)((rows + 63) / 64 * 64) * f.kp * 2) != EXN_OK) continue;   // the fp32 product then
     f.exact = true;
-    HIPCHK(vis_pack(s, rows, (int)cols, f.kp, std::ldexp(1.f, f.kw), v->t[e.name], f.h, rec + 4 * j + 2));
+    HIPCHK(vis_pack(s, rows, (int)cols, f.kp, std::ldexp(1.f, f.kw), v->t[e.name], f.h, rec + 4 * j + 1));
   }
   TRY(fetch());
   for (size_t j = 0; j < which.size(); ++j)
-    if (used(which[j]) && host[4 * j + 2]) v->facts[v->expect[which[j]].name].exact = false;
+    if (used(which[j]) && host[4 * j + 1]) v->facts[v->expect[which[j]].name].exact = false;
   return EXN_OK;
 }
 
-// the exponent that scales values of at most BOUND to at most 2^15; false where there is none
+// the exponent that scales values of at most BOUND to between 2^14 and 2^15; false where there is
+// none that the scales, their products and inverses hold as normal fp32 numbers
 static bool vis_exponent(double bound, int& e) {
   if (!(bound >= 0.0) || !std::isfinite(bound)) return false;
-  e = bound > 0.0 ? std::min(60, 14 - std::ilogb(bound * 1.01)) : 0;
-  return e >= -60;
+  e = bound > 0.0 ? 14 - std::ilogb(bound * 1.01) : 0;
+  return e >= -60 && e <= 60;
 }
 
 // The products of the tower and, from the weights alone, which of them run split and at which

@@ -340,10 +340,10 @@ hipError_t vis_attend(hipStream_t s, int n, int heads, const float* q, const flo
 hipError_t vis_sum(hipStream_t s, int64_t n, const float* a, const float* b, float* y);
 hipError_t round_f16(hipStream_t s, int64_t n, float* x);
 // ... and on fp16 parts of fp32 values (vision_split.hip): a split row is 2 KP halves, 32 hi then
-// 32 lo for every 32 columns.  vis_stats: the bits of max |x| and of the largest row's sum of
-// squares into rec[0], rec[1] (cleared first).  vis_pack: SCALE x as fp16 in the products'
-// order (KP/32 runs of rows rounded up to 64), *INEXACT set where a value changes.  vis_ln_s: X += BIAS + S parts (rows x width floats each), then
-// LayerNorm into YS (times SCALE) or fp32 YF.  vis_gemm_s: DESCALE X W^T + bias (+ R) into Y, or
+// 32 lo for every 32 columns.  vis_stats: the bits of max |x| into rec[0] and of the largest row's
+// sum of squares, a double, into rec[2], rec[3] (cleared first).  vis_pack: SCALE x as fp16 in the
+// products' order (KP/32 runs of rows rounded up to 64), *INEXACT set where a value changes.
+// vis_ln_s: X += BIAS + S parts (rows x width floats each), then LayerNorm into YS (times SCALE) or fp32 YF.  vis_gemm_s: DESCALE X W^T + bias (+ R) into Y, or
 // through GELU, times OSCALE, into split rows YS of LDY; vis_gemm_part: its S parts over K
 // (vis_split: how many pay).  vis_heads_s, vis_attend_s: heads and attention
 hipError_t vis_widen(hipStream_t s, int64_t n, const uint16_t* x, int bf16, float* y);   // 16-bit values as fp32

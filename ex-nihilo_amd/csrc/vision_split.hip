@@ -74,23 +74,29 @@ hipError_t vis_widen(hipStream_t s, int64_t n, const uint16_t* x, int bf16, floa
   return hipGetLastError();
 }
 
-// rec[0] = the bits of the largest |x|, rec[1] those of the largest row's sum of squares (NaNs
-// compare above every number, so a bound made from a tensor that holds one is not finite)
+// rec[0] = the bits of the largest |x|, rec[2] and rec[3] those of the largest row's sum of squares in
+// double, which no fp32 row makes 0 or infinite (NaNs compare above every number, so a bound made
+// from a tensor that holds one is not finite)
 __global__ void __launch_bounds__(256)
 k_vis_stats(int64_t rows, int64_t cols, const float* __restrict__ x, uint32_t* __restrict__ rec) {
   // a wave a row; one pair of atomics a workgroup (one a row took 100 us for 4304 rows)
-  __shared__ uint32_t rm[4], rs[4];
+  typedef unsigned long long u64;
+  __shared__ uint32_t rm[4];
+  __shared__ u64 rs[4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  uint32_t mb = 0u, sb = 0u;
+  uint32_t mb = 0u;
+  u64 sb = 0u;
   for (int64_t row = (int64_t)blockIdx.x * 4 + wave; row < rows; row += (int64_t)gridDim.x * 4) {
     const float* r = x + row * cols;
-    float s = 0.f;
+    double s = 0.0;
     for (int64_t i = lane; i < cols; i += 64) {
       const float v = r[i];
       mb = max(mb, __float_as_uint(fabsf(v)));
-      s += v * v;
+      s += (double)v * (double)v;
     }
-    sb = max(sb, __float_as_uint(fabsf(wave_sum(s))));
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    sb = max(sb, (u64)__double_as_longlong(fabs(s)));
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mb = max(mb, (uint32_t)__shfl_xor((int)mb, o, 64));
@@ -101,7 +107,7 @@ k_vis_stats(int64_t rows, int64_t cols, const float* __restrict__ x, uint32_t* _
   __syncthreads();
   if (threadIdx.x == 0) {
     atomicMax(rec, max(max(rm[0], rm[1]), max(rm[2], rm[3])));
-    atomicMax(rec + 1, max(max(rs[0], rs[1]), max(rs[2], rs[3])));
+    atomicMax((u64*)(rec + 2), max(max(rs[0], rs[1]), max(rs[2], rs[3])));
   }
 }
 

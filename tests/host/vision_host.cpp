@@ -5,7 +5,8 @@
 #include <cstdlib>
 
 static std::string g_err, g_log;
-static float g_max = 1.f, g_sumsq = 1.f;   // what vis_stats finds in the next tensors
+static float g_max = 1.f;   // what vis_stats finds in the next tensors
+static double g_sumsq = 1.0;
 static uint32_t g_inexact = 0;             // and vis_pack
 static int g_fail = 0;                     // vis_stats calls until one fails (0: none)
 static exn_ctx g_ctx;
@@ -31,7 +32,7 @@ hipError_t tensor_stats_clear(hipStream_t, uint32_t* rec, int64_t n) {
 hipError_t vis_stats(hipStream_t, int64_t, int64_t, const float*, uint32_t* rec) {
   if (g_fail && --g_fail == 0) return hipErrorUnknown;
   memcpy(rec, &g_max, 4);
-  memcpy(rec + 1, &g_sumsq, 4);
+  memcpy(rec + 2, &g_sumsq, 8);
   return hipSuccess;
 }
 hipError_t vis_pack(hipStream_t, int64_t, int, int, float, const float*, uint16_t*, uint32_t* inexact) {
@@ -97,7 +98,7 @@ hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "a planted failure"; }
 
 exn_ctx* vh_ctx() { return &g_ctx; }
-void vh_facts(float mx, float sumsq, int inexact, int fail) {
+void vh_facts(float mx, double sumsq, int inexact, int fail) {
   g_max = mx;
   g_sumsq = sumsq;
   g_inexact = (uint32_t)inexact;

@@ -224,6 +224,38 @@ def test_encode_with_split_and_fp32_products(ctx, owt, hw):
         v.destroy()
 
 
+def encode_edited(ctx, owt, edit, hw):
+    """A tower whose tensors are EDIT(name, values), its encode of a picture of HW and the oracle's;
+    relative L2 of block 0's rows, the merger's and the three deepstack sets."""
+    wt = vo.SynthVision(SEED, vo.VShape())
+    v = X.Vision(ctx)
+    try:
+        for name, shape in vo.vision_expected(vo.VShape()):
+            wt.cache[name] = np.asarray(edit(name, owt(name)), np.float32)
+            v.set(name, X.F32, wt.cache[name], shape)
+        px = vo.synth_picture(SEED + 9, *hw)
+        v.trace(True)
+        merged, deep, m = X.vision_encode(v, px, *hw)
+        want = vo.encode(px, wt)
+        return [xo.rel_l2(v.traced(1, 4 * m), want["blk0"]), xo.rel_l2(merged, want["merged"])] + \
+               [xo.rel_l2(deep[j], want["ds"][j]) for j in range(3)]
+    finally:
+        v.destroy()
+
+
+def test_encode_with_values_whose_squares_vanish(ctx, owt):
+    """Block 0's q | k | v 2^-75 of their size (their squares are zeros in fp32, their rows below
+    what the split heads' scales reach) and attn_out 2^75 times: the attention's part of the rows is
+    as large as before and as near to the oracle."""
+    def edit(name, a):
+        if name == "v.blk.0.attn_qkv.bias":
+            return 0 * a
+        return np.ldexp(a, -75 if name == "v.blk.0.attn_qkv.weight" else 75 if name == "v.blk.0.attn_out.weight" else 0)
+    errs = encode_edited(ctx, owt, edit, (64, 96))
+    say("squares vanish", errs)
+    assert errs[0] < 1e-5 and max(errs) < 1e-4
+
+
 def test_release_frees_scratch_and_keeps_weights(tower):
     """vision-release (src/cuda-vision.lisp:103-107): the scratch freed, the weights kept; the
     next encode makes its buffers again and gives the same rows bit for bit."""

@@ -28,7 +28,7 @@ def host(tmp_path_factory):
     L = ctypes.CDLL(so)
     L.vh_encode.restype = ctypes.c_char_p
     L.vh_ctx.restype = ctypes.c_void_p
-    L.vh_facts.argtypes = [ctypes.c_float, ctypes.c_float, ctypes.c_int, ctypes.c_int]
+    L.vh_facts.argtypes = [ctypes.c_float, ctypes.c_double, ctypes.c_int, ctypes.c_int]
     return L
 
 
@@ -114,3 +114,11 @@ def test_values_that_fp16_does_not_hold_run_in_fp32(tower):
 def test_bounds_that_are_not_finite_run_in_fp32(tower):
     assert tower.set("v.blk.0.ln1.bias", mx=float("nan"), norm=float("nan")) == OK
     assert tower.encode()[0][0] == BROKEN["ln1.weight"]
+
+
+def test_values_too_small_for_a_scale_run_in_fp32(tower):
+    """A q | k | v matrix of values near 2^-75 (no bias): no scale of at most 2^60 brings its rows to
+    where two fp16 parts hold them, and their norms are no zeros in fp32's own squares."""
+    assert tower.set("v.blk.2.attn_qkv.bias", mx=0.0, norm=0.0) == OK
+    assert tower.set("v.blk.2.attn_qkv.weight", mx=2.0 ** -75, norm=2.0 ** -71) == OK
+    assert tower.encode()[0][2] == SPLIT[:2] + ["heads/f", "attend/f", "mm/f"] + SPLIT[5:]
