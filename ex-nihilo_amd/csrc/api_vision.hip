@@ -149,6 +149,7 @@ static int vis_measure(exn_vision* v, const std::vector<size_t>& which) {
   TRY(vis_buf(v, "facts", v->expect.size() * 16, &recp));
   uint32_t* rec = (uint32_t*)recp;
   std::vector<uint32_t> host(which.size() * 4);
+  std::vector<bool> packed(which.size(), false);   // exact only once the flag has come back
   auto dims = [&](size_t i, int64_t& rows, int64_t& cols) {
     const std::vector<int64_t>& d = v->expect[i].shape;
     rows = d.size() > 1 ? d[0] : 1;
@@ -180,18 +181,17 @@ static int vis_measure(exn_vision* v, const std::vector<size_t>& which) {
     memcpy(&ss, &host[4 * j + 2], 8);
     f.mx = mx;
     f.norm = std::sqrt(ss) * 1.001;   // the sum's own rounding
-    f.exact = false;
     if (e.shape.size() < 2 || !std::isfinite(mx)) continue;
     dims(which[j], rows, cols);
     f.kp = (int)((cols + 63) / 64 * 64);
     f.kw = mx > 0.f ? std::min(40, std::max(0, 14 - std::ilogb(mx))) : 0;
     if (!f.h && dev_alloc((void**)&f.h, (size_t)((rows + 63) / 64 * 64) * f.kp * 2) != EXN_OK) continue;   // the fp32 product then
-    f.exact = true;
+    packed[j] = true;
     HIPCHK(vis_pack(s, rows, (int)cols, f.kp, std::ldexp(1.f, f.kw), v->t[e.name], f.h, rec + 4 * j + 1));
   }
   TRY(fetch());
   for (size_t j = 0; j < which.size(); ++j)
-    if (used(which[j]) && host[4 * j + 1]) v->facts[v->expect[which[j]].name].exact = false;
+    if (packed[j]) v->facts[v->expect[which[j]].name].exact = host[4 * j + 1] == 0;
   return EXN_OK;
 }
 

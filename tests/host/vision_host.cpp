@@ -8,7 +8,7 @@ static std::string g_err, g_log;
 static float g_max = 1.f;   // what vis_stats finds in the next tensors
 static double g_sumsq = 1.0;
 static uint32_t g_inexact = 0;             // and vis_pack
-static int g_fail = 0;                     // vis_stats calls until one fails (0: none)
+static int g_fail = 0;                     // the step that fails: 1 vis_stats, 2 vis_pack, 3 the flags' way back
 static exn_ctx g_ctx;
 
 namespace exn {
@@ -30,14 +30,15 @@ hipError_t tensor_stats_clear(hipStream_t, uint32_t* rec, int64_t n) {
   return hipSuccess;
 }
 hipError_t vis_stats(hipStream_t, int64_t, int64_t, const float*, uint32_t* rec) {
-  if (g_fail && --g_fail == 0) return hipErrorUnknown;
+  if (g_fail == 1) return hipErrorUnknown;
   memcpy(rec, &g_max, 4);
   memcpy(rec + 2, &g_sumsq, 8);
   return hipSuccess;
 }
 hipError_t vis_pack(hipStream_t, int64_t, int, int, float, const float*, uint16_t*, uint32_t* inexact) {
   *inexact = g_inexact;
-  return hipSuccess;
+  if (g_fail == 3) g_fail = -1;
+  return g_fail == 2 ? hipErrorUnknown : hipSuccess;
 }
 hipError_t vis_widen(hipStream_t, int64_t, const uint16_t*, int, float*) { return hipSuccess; }
 hipError_t round_f16(hipStream_t, int64_t, float*) { return hipSuccess; }
@@ -91,6 +92,7 @@ int ctx_tmp(exn_ctx* c, size_t n, void** out) {
 extern "C" {
 // only what comes back to the host is looked at
 hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind kind, hipStream_t) {
+  if (g_fail == -1) return hipErrorUnknown;
   if (kind == hipMemcpyDeviceToHost) memcpy(dst, src, n);
   return hipSuccess;
 }

@@ -39,7 +39,8 @@ class Tower:
         assert L.exn_vision_create(ctypes.c_void_p(L.vh_ctx()), ctypes.byref(self.h)) == OK
 
     def set(self, name, mx=1.0, norm=1.0, inexact=0, fail=0):
-        """Store tensor NAME; its measuring finds MX, NORM and INEXACT, or fails at its FAIL-th step."""
+        """Store tensor NAME; its measuring finds MX, NORM and INEXACT, or fails: 1 its
+        statistics, 2 a matrix's fp16 rows, 3 their flag's way back."""
         self.L.vh_facts(mx, norm * norm, inexact, fail)
         shape = self.shapes[name]
         return self.L.exn_vision_set(self.h, name.encode(), F32, DATA.ctypes.data_as(ctypes.c_void_p),
@@ -89,15 +90,18 @@ BROKEN = {   # the block's kernels without the tensor's facts
 }
 
 
-@pytest.mark.parametrize("tensor", list(BROKEN))
-def test_a_tensor_whose_measuring_failed_runs_in_fp32(tower, tensor):
+@pytest.mark.parametrize("tensor,fail", [(t, 1) for t in BROKEN] + [(t, f) for t in BROKEN if t.count("_") and "weight" in t
+                                         for f in (2, 3)])
+def test_a_tensor_whose_measuring_failed_runs_in_fp32(tower, tensor, fail):
     """A replaced tensor whose measuring fails has no fp16 rows and no bounds of its own: its product
     and those that its bounds reach run in fp32, the other blocks as before.  Measured again, all is
     as it was."""
     name = "v.blk.3." + tensor
-    assert tower.set(name, fail=1) != OK
+    assert tower.set(name, fail=fail) != OK
+    tower.L.vh_facts(1.0, 1.0, 0, 0)
     blocks, mergers = tower.encode()
-    assert blocks[3] == BROKEN[tensor]
+    # past step 1 the new values' bounds are known, so the attention on them may stay split
+    assert blocks[3] == (["ln/f", "mm/f"] + SPLIT[2:] if fail > 1 and tensor == "attn_qkv.weight" else BROKEN[tensor])
     assert blocks[:3] + blocks[4:] == [SPLIT] * 26 and mergers == [["ln/s", "mm/s", "mm/s"]] * 4
     assert tower.set(name) == OK
     assert tower.encode()[0] == [SPLIT] * 27
