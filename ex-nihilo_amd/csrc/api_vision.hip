@@ -87,11 +87,20 @@ struct VisMerger {
   VisMm fc1, fc2;
 };
 
+// A block (0 .. 26) or a merger (27 ..): for each of its products, in order, the largest
+// |w_j| / T_j (k_vis_rows), and q's and k's mean squares
+constexpr int kVisUnits = kVisDepth + 4;
+struct VisSpread {
+  double mm[4] = {INFINITY, INFINITY, INFINITY, INFINITY};
+  std::vector<double> qk;
+};
+
 struct exn_vision {
   exn_ctx* ctx = nullptr;
   std::vector<VExpect> expect;
   std::map<std::string, float*> t;   // fp32 device copies
   std::map<std::string, VisFacts> facts;
+  VisSpread spread[kVisUnits];
   std::vector<VisBlock> blocks;       // made from the weights when one changed
   VisMerger mergers[4];               // deepstack 0 .. 2, then the merger
   bool plan_ok = false;
@@ -128,11 +137,20 @@ static const float* vis_t(const exn_vision* v, const std::string& name) {
   return it == v->t.end() ? nullptr : it->second;
 }
 
+// the block or merger that reads tensor NAME; -1 the patch embedding
+static int vis_unit(const std::string& name) {
+  int i = 0;
+  if (sscanf(name.c_str(), "v.blk.%d.", &i) == 1) return i;
+  if (sscanf(name.c_str(), "v.deepstack.%d.", &i) == 1) return kVisDepth + (i - kVisDeep[0]) / 8;
+  return name.compare(0, 3, "mm.") == 0 || name.compare(0, 9, "v.post_ln") == 0 ? kVisUnits - 1 : -1;
+}
+
 // N fp32 values (device, DATA) into tensor NAME's device copy
 static int vis_store(exn_vision* v, const std::string& name, int64_t n, const float* data) {
   VisFacts& f = v->facts[name];   // the old values' go first: what follows may fail
   f.mx = f.norm = INFINITY;
   f.exact = false;
+  if (vis_unit(name) >= 0) v->spread[vis_unit(name)] = VisSpread();
   v->plan_ok = false;
   float*& p = v->t[name];
   if (!p) TRY(dev_alloc((void**)&p, (size_t)n * 4));
@@ -141,8 +159,65 @@ static int vis_store(exn_vision* v, const std::string& name, int64_t n, const fl
   return EXN_OK;
 }
 
+// UNITS' spreads, of those whose tensors are all there.  Ends with the stream idle.
+static int vis_spreads(exn_vision* v, const std::vector<int>& units) {
+  hipStream_t s = v->ctx->stream;
+  // a unit's doubles: 8 maxima, the outputs of its first product, then its inputs and other outputs
+  constexpr int64_t kOut = 8, kIn = kOut + 4608, kOther = kIn + 4608, kUnit = kOther + 4608;
+  double* buf = nullptr;
+  TRY(ctx_tmp(v->ctx, units.size() * kUnit * 8, (void**)&buf));
+  std::vector<int> done;
+  for (int u : units) {
+    double* m = buf + (int64_t)done.size() * kUnit;
+    bool all = true;
+    for (const VExpect& e : v->expect) all &= vis_unit(e.name) != u || vis_t(v, e.name);
+    if (!all) continue;
+    done.push_back(u);
+    char p[32];
+    if (u < kVisDepth) snprintf(p, sizeof p, "v.blk.%d.", u);
+    else if (u < kVisUnits - 1) snprintf(p, sizeof p, "v.deepstack.%d.", kVisDeep[u - kVisDepth]);
+    else p[0] = 0;
+    const std::string b = p;
+    auto square = [&](const std::string& name, int n) {
+      return vis_square(s, n, vis_t(v, name + ".weight"), vis_t(v, name + ".bias"), m + kIn);
+    };
+    auto rows = [&](const std::string& name, const double* in, int period, int gelu, double* out, int which) {
+      const VExpect* e = vis_find(v, (name + ".weight").c_str());
+      return vis_rows(s, (int)e->shape[0], (int)e->shape[1], vis_t(v, name + ".weight"), in, period,
+                      vis_t(v, name + ".bias"), gelu, out, m + which);
+    };
+    HIPCHK(tensor_stats_clear(s, (uint32_t*)m, 4));
+    if (u < kVisDepth) {
+      HIPCHK(square(b + "ln1", kVisD));
+      HIPCHK(rows(b + "attn_qkv", m + kIn, kVisD, 0, m + kOut, 0));
+      HIPCHK(rows(b + "attn_out", m + kOut + 2 * kVisD, kVisD, 0, m + kOther, 1));
+      HIPCHK(square(b + "ln2", kVisD));
+      HIPCHK(rows(b + "ffn_up", m + kIn, kVisD, 1, m + kOther, 2));
+      HIPCHK(rows(b + "ffn_down", m + kOther, kVisF, 0, m + kIn, 3));
+    } else {
+      const bool last = u == kVisUnits - 1;
+      const int width = last ? kVisD : 4 * kVisD;
+      HIPCHK(square(last ? "v.post_ln" : b + "norm", width));
+      HIPCHK(rows(last ? "mm.0" : b + "fc1", m + kIn, width, 1, m + kOther, 0));
+      HIPCHK(rows(last ? "mm.2" : b + "fc2", m + kOther, 4 * kVisD, 0, m + kOut, 1));
+    }
+  }
+  std::vector<double> host(done.size() * (size_t)(8 + 2 * kVisD));
+  for (size_t i = 0; i < done.size(); ++i)
+    HIPCHK(hipMemcpyAsync(&host[i * (8 + 2 * kVisD)], buf + (int64_t)i * kUnit, (8 + 2 * kVisD) * 8, hipMemcpyDeviceToHost, s));
+  HIPCHK(hipStreamSynchronize(s));
+  for (size_t i = 0; i < done.size(); ++i) {
+    const double* m = &host[i * (8 + 2 * kVisD)];
+    VisSpread& r = v->spread[done[i]];
+    for (int k = 0; k < 4; ++k) r.mm[k] = std::sqrt(m[k]);
+    r.qk.assign(m + 8, m + 8 + 2 * kVisD);
+  }
+  return EXN_OK;
+}
+
 // the facts of the stored tensors WHICH (indices of expect): two passes over each on the device,
-// the second, where the values fit, the fp16 rows.  Ends with the stream idle.
+// the second, where the values fit, the fp16 rows; then their units' spreads.  Ends with the stream
+// idle.
 static int vis_measure(exn_vision* v, const std::vector<size_t>& which) {
   hipStream_t s = v->ctx->stream;
   float* recp = nullptr;
@@ -192,7 +267,12 @@ static int vis_measure(exn_vision* v, const std::vector<size_t>& which) {
   TRY(fetch());
   for (size_t j = 0; j < which.size(); ++j)
     if (packed[j]) v->facts[v->expect[which[j]].name].exact = host[4 * j + 1] == 0;
-  return EXN_OK;
+  std::vector<int> units;
+  for (size_t i : which) {
+    const int u = vis_unit(v->expect[i].name);
+    if (u >= 0 && std::find(units.begin(), units.end(), u) == units.end()) units.push_back(u);
+  }
+  return vis_spreads(v, units);
 }
 
 // the exponent that scales values of at most BOUND to between 2^14 and 2^15; false where there is
@@ -201,6 +281,36 @@ static bool vis_exponent(double bound, int& e) {
   if (!(bound >= 0.0) || !std::isfinite(bound)) return false;
   e = bound > 0.0 ? 14 - std::ilogb(bound * 1.01) : 0;
   return e >= -60 && e <= 60;
+}
+
+// A split value is off by up to 2^-40 of the bound B that its scale was made for, whatever its own
+// size, so that a product's output j is off by up to about 2^-40 B |w_j|, and where B is far above
+// what most inputs have (one LayerNorm gain or weight row far above the others, taken back by the
+// next matrix's column) that passes fp32's own rounding.  Split where it is at most 2^-23 of every
+// output's own size T_j: B |w_j| / T_j up to 2^17.  Of 1152 inputs one 2^12 times the others, at that
+// limit: rounded to the split's parts a product is 1.4e-7 off, its fp32 sums 3.1e-7; 2^16 times: 2.2e-6.
+// Normally distributed weights stand at 2^6.
+constexpr double kVisSpread = 1 << 17;
+// attention's output may be as small as its values over 64, where 4096 patches weigh alike
+constexpr double kVisSpreadAtt = kVisSpread / 64;
+
+// the same of a score, sum q k over a head: its error against its own size, or against 1 where it is
+// smaller (exp2's input)
+static bool vis_heads_fit(const std::vector<double>& qk, double bq, double bk) {
+  if (qk.empty()) return false;
+  const double qs = 1.4426950408889634 / std::sqrt((double)kVisHd);
+  for (int h = 0; h < kVisHeads; ++h) {
+    double q2 = 0, k2 = 0, s2 = 0;
+    for (int d = 0; d < kVisHd; ++d) {
+      const int at = h * kVisHd + d, to = h * kVisHd + (d + kVisHd / 2) % kVisHd;   // the rotary turns the two into each other
+      const double q = 0.5 * (qk[at] + qk[to]) * qs * qs, k = 0.5 * (qk[kVisD + at] + qk[kVisD + to]);
+      q2 += q;
+      k2 += k;
+      s2 += q * k;
+    }
+    if (!(bq * std::sqrt(k2) + bk * std::sqrt(q2) <= kVisSpread * std::max(1.0, std::sqrt(s2)))) return false;
+  }
+  return true;
 }
 
 // The products of the tower and, from the weights alone, which of them run split and at which
@@ -232,7 +342,7 @@ static void vis_plan(exn_vision* v) {
     return Bound{r + b.mx, r + b.norm};
   };
   auto out = [&](const std::string& name, double norm) { return norm * facts(name + ".weight").norm + facts(name + ".bias").mx; };
-  auto merger = [&](const std::string& norm, const std::string& fc1, const std::string& fc2, int width) {
+  auto merger = [&](const std::string& norm, const std::string& fc1, const std::string& fc2, int width, const VisSpread& sp) {
     VisMerger m;
     m.lnw = vis_t(v, norm + ".weight");
     m.lnb = vis_t(v, norm + ".bias");
@@ -240,7 +350,8 @@ static void vis_plan(exn_vision* v) {
     m.fc2 = mm(fc2);
     const Bound z = ln(norm, width);
     const double rn = z.norm * std::sqrt(m.fc1.k / (double)width);   // the row is k / width normed ones
-    const bool ok = m.fc1.split && m.fc2.split && vis_exponent(z.el, m.fc1.ex) && vis_exponent(out(fc1, rn), m.fc2.ex);
+    const bool ok = m.fc1.split && m.fc2.split && vis_exponent(z.el, m.fc1.ex) && vis_exponent(out(fc1, rn), m.fc2.ex) &&
+                    z.el * sp.mm[0] <= kVisSpread && out(fc1, rn) * sp.mm[1] <= kVisSpread;
     m.fc1.split = m.fc2.split = ok;
     return m;
   };
@@ -259,23 +370,26 @@ static void vis_plan(exn_vision* v) {
     k.up = mm(b + "ffn_up");
     k.down = mm(b + "ffn_down");
     const Bound z1 = ln(b + "ln1", kVisD), z2 = ln(b + "ln2", kVisD);
-    const double head = out(b + "attn_qkv", z1.norm);
-    k.qkv.split = k.qkv.split && vis_exponent(z1.el, k.qkv.ex);
-    k.heads = vis_exponent(head * 1.4143 * 1.4427 / std::sqrt((double)kVisHd), k.eq) &&
-              vis_exponent(head * 1.4143, k.ek) && vis_exponent(head, k.ev);
+    const VisSpread& sp = v->spread[i];
+    const double head = out(b + "attn_qkv", z1.norm), up = out(b + "ffn_up", z2.norm);
+    const double bq = head * 1.4143 * 1.4427 / std::sqrt((double)kVisHd), bk = head * 1.4143;
+    k.qkv.split = k.qkv.split && vis_exponent(z1.el, k.qkv.ex) && z1.el * sp.mm[0] <= kVisSpread;
+    // V's parts are averaged as V is, so that they ask what attn_out asks of the averages
+    k.heads = vis_exponent(bq, k.eq) && vis_exponent(bk, k.ek) && vis_exponent(head, k.ev) &&
+              vis_heads_fit(sp.qk, bq, bk) && head * sp.mm[1] <= kVisSpread;
     k.out.ex = k.ev;
-    k.out.split = k.out.split && k.heads;
-    const bool ok = k.up.split && k.down.split && vis_exponent(z2.el, k.up.ex) &&
-                    vis_exponent(out(b + "ffn_up", z2.norm), k.down.ex);
+    k.out.split = k.out.split && k.heads && head * sp.mm[1] <= kVisSpreadAtt;
+    const bool ok = k.up.split && k.down.split && vis_exponent(z2.el, k.up.ex) && vis_exponent(up, k.down.ex) &&
+                    z2.el * sp.mm[2] <= kVisSpread && up * sp.mm[3] <= kVisSpread;
     k.up.split = k.down.split = ok;
     v->blocks.push_back(k);
   }
   for (int j = 0; j < 3; ++j) {
     snprintf(p, sizeof p, "v.deepstack.%d", kVisDeep[j]);
     const std::string b = p;
-    v->mergers[j] = merger(b + ".norm", b + ".fc1", b + ".fc2", 4 * kVisD);
+    v->mergers[j] = merger(b + ".norm", b + ".fc1", b + ".fc2", 4 * kVisD, v->spread[kVisDepth + j]);
   }
-  v->mergers[3] = merger("v.post_ln", "mm.0", "mm.2", kVisD);
+  v->mergers[3] = merger("v.post_ln", "mm.0", "mm.2", kVisD, v->spread[kVisUnits - 1]);
   v->plan_ok = true;
 }
 

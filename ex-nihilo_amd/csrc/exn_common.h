@@ -350,6 +350,11 @@ hipError_t vis_widen(hipStream_t s, int64_t n, const uint16_t* x, int bf16, floa
 hipError_t vis_stats(hipStream_t s, int64_t rows, int64_t cols, const float* x, uint32_t* rec);
 hipError_t vis_pack(hipStream_t s, int64_t rows, int K, int KP, float scale, const float* x, uint16_t* y,
                     uint32_t* inexact);
+// vis_square, vis_rows: the sizes that inputs and outputs have where rows have no structure, from the
+// weights (doubles), for the tower's plan
+hipError_t vis_square(hipStream_t s, int n, const float* g, const float* b, double* a2);
+hipError_t vis_rows(hipStream_t s, int rows, int cols, const float* w, const double* a2, int period, const float* bias,
+                    int gelu, double* t2, double* spread);
 hipError_t vis_ln_s(hipStream_t s, int64_t rows, int width, int kp, float* x, int S, const float* part,
                     const float* bias, const float* w, const float* b, float scale, uint16_t* ys, float* yf);
 hipError_t vis_gemm_s(hipStream_t s, const uint16_t* x, const uint16_t* w, const float* bias, const float* r, float* y,

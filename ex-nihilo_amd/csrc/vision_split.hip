@@ -144,6 +144,64 @@ hipError_t vis_pack(hipStream_t s, int64_t rows, int K, int KP, float scale, con
   return hipGetLastError();
 }
 
+// a2[i] = g[i]^2 + b[i]^2: the mean square of a LayerNorm's output i over rows of no structure
+__global__ void k_vis_square(int n, const float* __restrict__ g, const float* __restrict__ b, double* __restrict__ a2) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) a2[i] = (double)g[i] * g[i] + (double)b[i] * b[i];
+}
+
+hipError_t vis_square(hipStream_t s, int n, const float* g, const float* b, double* a2) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_vis_square, dim3(sgrid(n, 256)), dim3(256), 0, s, n, g, b, a2);
+  return hipGetLastError();
+}
+
+__device__ __forceinline__ double gelu_d(double x) { return 0.5 * x * (1.0 + erf(x * 0.70710678118654752)); }
+
+// For inputs of mean squares a2 (PERIOD of them, over and over along a row) without structure: t2[j],
+// the mean square of W's output j (its deviation T_j about the bias), or of its GELU (three points
+// of the normal distribution, exact for polynomials of degree 5), and *SPREAD, the bits of the
+// largest |w_j|^2 / T_j^2: how much larger than an output's own size the error of a step of 1 in
+// every input is.  A wave a row, sums in double.
+__global__ void __launch_bounds__(256)
+k_vis_rows(int rows, int cols, const float* __restrict__ w, const double* __restrict__ a2, int period,
+           const float* __restrict__ bias, int gelu, double* __restrict__ t2, unsigned long long* spread) {
+  const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const float* r = w + (int64_t)row * cols;
+  double q = 0.0, t = 0.0;
+  // COLS and PERIOD are multiples of 4: a lane's four columns never cross a period's end
+  for (int i = 4 * lane, p = i; i < cols; i += 256, p += 256) {
+    while (p >= period) p -= period;
+    const f32x4 x = *(const f32x4*)(r + i);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const double v = (double)x[e] * x[e];
+      q += v;
+      t += v * a2[p + e];
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    q += __shfl_xor(q, o, 64);
+    t += __shfl_xor(t, o, 64);
+  }
+  if (lane) return;
+  const double b = bias[row], d = 1.7320508075688772 * sqrt(t);
+  const double lo = gelu_d(b - d), md = gelu_d(b), hi = gelu_d(b + d);
+  t2[row] = gelu ? (lo * lo + 4.0 * md * md + hi * hi) / 6.0 : t + b * b;
+  if (q != 0.0) atomicMax(spread, (unsigned long long)__double_as_longlong(fabs(q / t)));   // a row of zeros has no error
+}
+
+hipError_t vis_rows(hipStream_t s, int rows, int cols, const float* w, const double* a2, int period, const float* bias,
+                    int gelu, double* t2, double* spread) {
+  if (rows <= 0 || cols <= 0) return hipSuccess;
+  if (cols % 4 || period % 4 || period <= 0 || ((uintptr_t)w & 15)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_vis_rows, dim3(sgrid(rows, 4)), dim3(256), 0, s, rows, cols, w, a2, period, bias, gelu, t2,
+                     (unsigned long long*)spread);
+  return hipGetLastError();
+}
+
 // --- LayerNorm -------------------------------------------------------------------------------
 
 // One workgroup a row of WIDTH (a multiple of 4, at most 5120) of X, or, when S > 0, of

@@ -8,7 +8,9 @@ static std::string g_err, g_log;
 static float g_max = 1.f;   // what vis_stats finds in the next tensors
 static double g_sumsq = 1.0;
 static uint32_t g_inexact = 0;             // and vis_pack
-static int g_fail = 0;                     // the step that fails: 1 vis_stats, 2 vis_pack, 3 the flags' way back
+static int g_fail = 0;                     // the step that fails: 1 vis_stats, 2 vis_pack, 3 the flags' way back, 4 vis_rows
+static int g_rows = 0, g_cols = 0;         // the product (its W's shape) of spread g_spread; the others' is 1
+static double g_spread = 1.0, g_qk = 1.0;  // and q's and k's mean squares
 static exn_ctx g_ctx;
 
 namespace exn {
@@ -39,6 +41,13 @@ hipError_t vis_pack(hipStream_t, int64_t, int, int, float, const float*, uint16_
   *inexact = g_inexact;
   if (g_fail == 3) g_fail = -1;
   return g_fail == 2 ? hipErrorUnknown : hipSuccess;
+}
+hipError_t vis_square(hipStream_t, int, const float*, const float*, double*) { return hipSuccess; }
+hipError_t vis_rows(hipStream_t, int rows, int cols, const float*, const double*, int, const float*, int, double* t2, double* spread) {
+  for (int i = 0; i < rows; ++i) t2[i] = g_qk;
+  if (g_fail == 4) return hipErrorUnknown;
+  *spread = rows == g_rows && cols == g_cols ? g_spread * g_spread : 1.0;
+  return hipSuccess;
 }
 hipError_t vis_widen(hipStream_t, int64_t, const uint16_t*, int, float*) { return hipSuccess; }
 hipError_t round_f16(hipStream_t, int64_t, float*) { return hipSuccess; }
@@ -105,6 +114,12 @@ void vh_facts(float mx, double sumsq, int inexact, int fail) {
   g_sumsq = sumsq;
   g_inexact = (uint32_t)inexact;
   g_fail = fail;
+}
+void vh_spread(int rows, int cols, double spread, double qk) {
+  g_rows = rows;
+  g_cols = cols;
+  g_spread = spread;
+  g_qk = qk;
 }
 // the kernels an encode of a 64 x 64 picture launches, in order
 const char* vh_encode(exn_vision* v) {

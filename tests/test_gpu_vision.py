@@ -256,6 +256,55 @@ def test_encode_with_values_whose_squares_vanish(ctx, owt):
     assert errs[0] < 1e-5 and max(errs) < 1e-4
 
 
+def _to_f16(a):
+    return a.astype(np.float16).astype(np.float32)
+
+
+def _outlier(kind):
+    """EDIT for encode_edited: one of block 0's values 2^16 to 2^20 times the others, taken back
+    by the matrix behind it, whose column then holds fp16 values near its smallest."""
+    def edit(name, a):
+        a = np.array(a, np.float32)
+        if kind == "gain":
+            if name in ("v.blk.0.ln1.weight", "v.blk.0.ln2.weight"):
+                a[100] *= 2 ** 20
+            elif name in ("v.blk.0.attn_qkv.weight", "v.blk.0.ffn_up.weight"):
+                a[:, 100] = _to_f16(a[:, 100] / 2 ** 20)
+        elif kind == "value":
+            if name.startswith("v.blk.0.attn_qkv."):
+                a[2 * 1152 + 300] *= 2 ** 16
+            elif name == "v.blk.0.attn_out.weight":
+                a[:, 300] = _to_f16(a[:, 300] / 2 ** 16)
+        elif kind == "unit":
+            if name.startswith("v.blk.0.ffn_up."):
+                a[700] *= 2 ** 18
+            elif name == "v.blk.0.ffn_down.weight":
+                a[:, 700] = _to_f16(a[:, 700] / 2 ** 18)
+        elif kind == "query" and name.startswith("v.blk.0.attn_qkv."):
+            for d in (5, 41):                    # a pair that the rotary turns, of head 3's q and k
+                a[3 * 72 + d] *= 2 ** 16
+                a[1152 + 3 * 72 + d] = _to_f16(a[1152 + 3 * 72 + d] / 2 ** 16)
+        elif kind == "merger":
+            if name == "v.post_ln.weight":
+                a[100] *= 2 ** 20
+            elif name == "mm.0.weight":
+                a[:, 100::1152] = _to_f16(a[:, 100::1152] / 2 ** 20)
+        return a
+    return edit
+
+
+@pytest.mark.parametrize("kind", ["gain", "value", "unit", "query", "merger"])
+def test_encode_with_outliers(ctx, owt, kind):
+    """One LayerNorm gain, V row, MLP unit, q and k pair or merger gain far above the others and taken
+    back by the next matrix: the scale that the split products' bound asks for leaves the other
+    values too few bits, so those products run in fp32, and the distance from the oracle is at most
+    twice that of the ordinary tower with a block in fp32 (block 0's rows 1.3e-6, the merger's 2.4e-5).
+    Split they are 4e-6 to 1.4e-2 off after block 0 (a merger 1.1e-4)."""
+    errs = encode_edited(ctx, owt, _outlier(kind), (64, 96))
+    say("outlier", kind, errs)
+    assert errs[0] < 2.6e-6 and max(errs) < 4.8e-5
+
+
 def test_release_frees_scratch_and_keeps_weights(tower):
     """vision-release (src/cuda-vision.lisp:103-107): the scratch freed, the weights kept; the
     next encode makes its buffers again and gives the same rows bit for bit."""
