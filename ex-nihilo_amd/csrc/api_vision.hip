@@ -730,8 +730,67 @@ int exn_vis_attend(exn_ctx* ctx, int n, int heads, const float* q, const float* 
 int exn_vis_ln(exn_ctx* ctx, int64_t rows, int width, const float* x, const float* w, const float* b, float* y) {
   TRY(use(ctx));
   if (!x || !w || !b || !y || rows < 0) FAIL(EXN_EINVAL, "vis ln arguments");
-  const hipError_t e = vis_ln(ctx->stream, rows, width, x, w, b, y);
+  const hipError_t e = vis_ln_s(ctx->stream, rows, width, 0, (float*)x, 0, nullptr, nullptr, w, b, 1.f, nullptr, y);
   if (e == hipErrorInvalidValue) FAIL(EXN_EINVAL, "vis ln: width %d (a multiple of 4, at most 5120)", width);
   HIPCHK(e);
+  return EXN_OK;
+}
+
+int exn_vis_gemm_way(int64_t m, int64_t n, int64_t kp, int parts, int* tile, int* pays) {
+  if (!tile || !pays || m <= 0 || n <= 0 || kp < 64 || kp % 64 || parts < 1 || parts > kp / 64)
+    FAIL(EXN_EINVAL, "vis gemm way arguments");
+  *tile = vis_tile(m, n, kp, parts);
+  *pays = vis_split(m, n, kp);
+  return EXN_OK;
+}
+
+int exn_vis_gemm_s(exn_ctx* ctx, const uint16_t* x, const uint16_t* w, const float* bias, const float* r, float* y,
+                   uint16_t* ys, int64_t m, int64_t n, int64_t kp, float descale, float oscale, int64_t ldy, int act,
+                   int parts) {
+  TRY(use(ctx));
+  if (!x || !w || !y == !ys || parts < 1 || (parts > 1 ? !y || r || act : !bias)) FAIL(EXN_EINVAL, "vis gemm_s arguments");
+  const hipError_t e = parts > 1 ? vis_gemm_part(ctx->stream, x, w, y, m, n, kp, descale, parts)
+                                 : vis_gemm_s(ctx->stream, x, w, bias, r, y, ys, m, n, kp, descale, oscale, ldy, act);
+  if (e == hipErrorInvalidValue)
+    FAIL(EXN_EINVAL, "vis gemm_s: %lld x %lld x %lld, %d parts", (long long)m, (long long)n, (long long)kp, parts);
+  HIPCHK(e);
+  return EXN_OK;
+}
+
+int exn_vis_ln_s(exn_ctx* ctx, int64_t rows, int width, float* x, int parts, const float* part, const float* bias,
+                 const float* w, const float* b, float scale, uint16_t* ys, float* yf) {
+  TRY(use(ctx));
+  if (!x || !w || !b || rows < 0 || (parts > 0 && (!part || !bias))) FAIL(EXN_EINVAL, "vis ln_s arguments");
+  const hipError_t e = vis_ln_s(ctx->stream, rows, width, width, x, parts, part, bias, w, b, scale, ys, yf);
+  if (e == hipErrorInvalidValue) FAIL(EXN_EINVAL, "vis ln_s: width %d (a multiple of 64, at most 5120)", width);
+  HIPCHK(e);
+  return EXN_OK;
+}
+
+int exn_vis_heads_s(exn_ctx* ctx, int n, int heads, const float* qkv, const float* cs, float qs, float ks, float vs,
+                    uint16_t* q, uint16_t* k, uint16_t* vt) {
+  TRY(use(ctx));
+  if (!qkv || !cs || !q || !k || !vt || n <= 0 || heads <= 0) FAIL(EXN_EINVAL, "vis heads_s arguments");
+  HIPCHK(vis_heads_s(ctx->stream, n, (n + 63) / 64 * 64, heads, qkv, cs, qs, ks, vs, q, k, vt));
+  return EXN_OK;
+}
+
+int exn_vis_attend_s(exn_ctx* ctx, int n, int heads, const uint16_t* q, const uint16_t* k, const uint16_t* vt, float sc,
+                     float vde, uint16_t* ys, float* yf) {
+  TRY(use(ctx));
+  if (!q || !k || !vt || !ys == !yf || n <= 0 || heads <= 0 || (ys && heads * 72 % 64))
+    FAIL(EXN_EINVAL, "vis attend_s arguments");
+  HIPCHK(vis_attend_s(ctx->stream, n, (n + 63) / 64 * 64, heads, q, k, vt, sc, vde, heads * 72, ys, yf));
+  return EXN_OK;
+}
+
+int exn_vis_spread(exn_ctx* ctx, int rows, int cols, const float* w, const float* g, const float* b, int period,
+                   const float* bias, int gelu, double* a2, double* t2, double* spread2) {
+  TRY(use(ctx));
+  if (!w || !g || !b || !bias || !a2 || !t2 || !spread2 || rows <= 0 || cols <= 0 || cols % 4 || period <= 0 || period % 4)
+    FAIL(EXN_EINVAL, "vis spread arguments");
+  HIPCHK(tensor_stats_clear(ctx->stream, (uint32_t*)spread2, 1));
+  HIPCHK(vis_square(ctx->stream, period, g, b, a2));
+  HIPCHK(vis_rows(ctx->stream, rows, cols, w, a2, period, bias, gelu, t2, spread2));
   return EXN_OK;
 }

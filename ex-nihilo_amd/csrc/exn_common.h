@@ -331,7 +331,6 @@ hipError_t vae_round_bf16(hipStream_t s, int64_t n, float* x);
 // Y = X W^T + bias (+ R) (act 0 none, 1 GELU tanh, 2 GELU erf), heads with the rotary, attention
 hipError_t vis_prep(hipStream_t s, const float* px, int w, int gh, int gw, const float* table, int side, int D,
                     float* pat, float* pe, float* cs);
-hipError_t vis_ln(hipStream_t s, int64_t rows, int width, const float* x, const float* w, const float* b, float* y);
 hipError_t vis_gemm(hipStream_t s, const float* x, const float* w, const float* bias, const float* r, float* y,
                     int64_t M, int64_t N, int64_t K, int act);
 hipError_t vis_heads(hipStream_t s, int n, int heads, const float* qkv, const float* cs, float qscale, float* q,
@@ -360,6 +359,7 @@ hipError_t vis_ln_s(hipStream_t s, int64_t rows, int width, int kp, float* x, in
 hipError_t vis_gemm_s(hipStream_t s, const uint16_t* x, const uint16_t* w, const float* bias, const float* r, float* y,
                       uint16_t* ys, int64_t M, int64_t N, int64_t KP, float descale, float oscale, int64_t ldy, int act);
 int vis_split(int64_t M, int64_t N, int64_t KP);
+int vis_tile(int64_t M, int64_t N, int64_t KP, int S);   // which of the product's tiles runs (0 .. 6)
 hipError_t vis_gemm_part(hipStream_t s, const uint16_t* x, const uint16_t* w, float* part, int64_t M, int64_t N,
                          int64_t KP, float descale, int S);
 hipError_t vis_heads_s(hipStream_t s, int n, int np, int heads, const float* qkv, const float* cs, float qs, float ks,

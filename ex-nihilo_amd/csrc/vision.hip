@@ -6,7 +6,6 @@
 //                 bilinearly from the table and the 2-D rotary's cosines and sines
 //                 (src/host.lisp:119-166, which the reference runs on the host);
 //   k_vis_gemm    Y = X W^T + b (+ R) (then GELU), fp32 products on v_mfma_f32_16x16x4_f32;
-//   k_vis_ln      LayerNorm rows, eps 1e-6;
 //   k_vis_heads   QKV rows into heads: q and k turned by the rotary, q scaled for the exp2
 //                 softmax, V transposed;
 //   k_vis_attend  softmax attention of every patch over every patch, flash-style, fp32 MFMAs.
@@ -105,64 +104,6 @@ hipError_t vis_prep(hipStream_t s, const float* px, int w, int gh, int gw, const
   const int n = gh * gw;
   if (n <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_vis_prep, dim3(n), dim3(256), 0, s, px, w, gh, gw, table, side, D, pat, pe, cs);
-  return hipGetLastError();
-}
-
-// --- LayerNorm ----------------------------------------------------------------------------
-
-// one workgroup a row of WIDTH (a multiple of 4, at most 5120): mean, then the mean square about
-// it, (x - mean) / sqrt(var + eps) * w + b, as inspect/ref_vision.py:35-38 orders it
-__global__ void __launch_bounds__(256)
-k_vis_ln(int width, const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ b,
-         float* __restrict__ y) {
-#pragma clang fp contract(off)
-  __shared__ float red[2][4];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, w4 = width >> 2;
-  const f32x4* r = (const f32x4*)(x + (int64_t)blockIdx.x * width);
-  f32x4 v[5];
-  float s = 0.f;
-#pragma unroll
-  for (int e = 0; e < 5; ++e) {
-    const int i = t + 256 * e;
-    v[e] = i < w4 ? r[i] : f32x4{0.f, 0.f, 0.f, 0.f};
-    s += (v[e][0] + v[e][1]) + (v[e][2] + v[e][3]);
-  }
-  s = wave_sum(s);
-  if (lane == 0) red[0][wave] = s;
-  __syncthreads();
-  const float mean = ((red[0][0] + red[0][1]) + (red[0][2] + red[0][3])) / (float)width;
-  float q = 0.f;
-#pragma unroll
-  for (int e = 0; e < 5; ++e)
-    if (t + 256 * e < w4)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float d = v[e][j] - mean;
-        q += d * d;
-      }
-  q = wave_sum(q);
-  if (lane == 0) red[1][wave] = q;
-  __syncthreads();
-  const float var = ((red[1][0] + red[1][1]) + (red[1][2] + red[1][3])) / (float)width;
-  const float sd = __fsqrt_rn(var + 1e-6f);
-  f32x4* o = (f32x4*)(y + (int64_t)blockIdx.x * width);
-#pragma unroll
-  for (int e = 0; e < 5; ++e) {
-    const int i = t + 256 * e;
-    if (i < w4) {
-      const f32x4 g = ((const f32x4*)w)[i], bb = ((const f32x4*)b)[i];
-      f32x4 z;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) z[j] = __fdiv_rn(v[e][j] - mean, sd) * g[j] + bb[j];
-      o[i] = z;
-    }
-  }
-}
-
-hipError_t vis_ln(hipStream_t s, int64_t rows, int width, const float* x, const float* w, const float* b, float* y) {
-  if (rows <= 0) return hipSuccess;
-  if (width % 4 || width > 5120) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_vis_ln, dim3((unsigned)rows), dim3(256), 0, s, width, x, w, b, y);
   return hipGetLastError();
 }
 

@@ -206,8 +206,9 @@ hipError_t vis_rows(hipStream_t s, int rows, int cols, const float* w, const dou
 
 // One workgroup a row of WIDTH (a multiple of 4, at most 5120) of X, or, when S > 0, of
 // bias + R + the S parts of a split product (each MN floats after the last, summed in order),
-// written back to X; then k_vis_ln's LayerNorm, times SCALE, into split rows of KP, or, when YF
-// is given, as fp32 rows.
+// written back to X; then LayerNorm (the mean, the mean square about it, (x - mean) /
+// sqrt(var + 1e-6) w + b, as inspect/ref_vision.py:35-38 orders it), times SCALE, into split rows of
+// KP, or, when YF is given, as fp32 rows.
 __global__ void __launch_bounds__(256)
 k_vis_ln_s(int width, int kp, float* __restrict__ x, int S, int64_t mn, const float* __restrict__ part,
            const float* __restrict__ bias, const float* __restrict__ w, const float* __restrict__ b, float scale,
@@ -275,7 +276,8 @@ k_vis_ln_s(int width, int kp, float* __restrict__ x, int S, int64_t mn, const fl
 hipError_t vis_ln_s(hipStream_t s, int64_t rows, int width, int kp, float* x, int S, const float* part,
                     const float* bias, const float* w, const float* b, float scale, uint16_t* ys, float* yf) {
   if (rows <= 0) return hipSuccess;
-  if (width % 64 || width > 5120 || kp != width) return hipErrorInvalidValue;   // no columns past the width to clear
+  if (width <= 0 || width % 4 || width > 5120 || S < 0 || !ys == !yf) return hipErrorInvalidValue;
+  if (ys && (width % 64 || kp != width)) return hipErrorInvalidValue;   // no columns past the width to clear
   hipLaunchKernelGGL(k_vis_ln_s, dim3((unsigned)rows), dim3(256), 0, s, width, kp, x, S, rows * width, part, bias, w, b,
                      scale, ys, yf);
   return hipGetLastError();
@@ -531,6 +533,11 @@ hipError_t vis_gemm_s(hipStream_t s, const uint16_t* x, const uint16_t* w, const
   if (act == 1)
     return gemm_s_tile<VS_SPLIT, 1>(s, x, w, bias, nullptr, ys, (int)M, (int)N, (int)KP, descale, oscale, (int)ldy, 1);
   return gemm_s_tile<VS_SPLIT, 2>(s, x, w, bias, nullptr, ys, (int)M, (int)N, (int)KP, descale, oscale, (int)ldy, 1);
+}
+
+int vis_tile(int64_t M, int64_t N, int64_t KP, int S) {
+  float cost;
+  return best_tile(M, N, KP, S, &cost);
 }
 
 // S parts cost a k-step's share each, the parts' store and the LayerNorm's reads (8 bytes a value

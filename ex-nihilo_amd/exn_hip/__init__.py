@@ -135,6 +135,13 @@ SIGNATURES = {
     "exn_vis_gemm": (c_int, [vp, vp, vp, vp, vp, vp, c_int64, c_int64, c_int64, c_int]),
     "exn_vis_attend": (c_int, [vp, c_int, c_int, vp, vp, vp, vp]),
     "exn_vis_ln": (c_int, [vp, c_int64, c_int, vp, vp, vp, vp]),
+    "exn_vis_gemm_way": (c_int, [c_int64, c_int64, c_int64, c_int, vp, vp]),
+    "exn_vis_gemm_s": (c_int, [vp, vp, vp, vp, vp, vp, vp, c_int64, c_int64, c_int64, c_float, c_float, c_int64, c_int,
+                               c_int]),
+    "exn_vis_ln_s": (c_int, [vp, c_int64, c_int, vp, c_int, vp, vp, vp, vp, c_float, vp, vp]),
+    "exn_vis_heads_s": (c_int, [vp, c_int, c_int, vp, vp, c_float, c_float, c_float, vp, vp, vp]),
+    "exn_vis_attend_s": (c_int, [vp, c_int, c_int, vp, vp, vp, c_float, c_float, vp, vp]),
+    "exn_vis_spread": (c_int, [vp, c_int, c_int, vp, vp, vp, c_int, vp, c_int, vp, vp, vp]),
     "exn_dit_stats": (c_int, [vp, c_int]),
     "exn_dit_stats_read": (c_int, [vp, vp, vp, c_int64]),
     "exn_enc_create": (c_int, [vp, c_int, c_double, POINTER(vp)]),

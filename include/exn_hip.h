@@ -370,6 +370,34 @@ int exn_vis_gemm(exn_ctx* ctx, const float* x, const float* w, const float* bias
                  int64_t n, int64_t k, int act);
 int exn_vis_attend(exn_ctx* ctx, int n, int heads, const float* q, const float* k, const float* vt, float* att);
 int exn_vis_ln(exn_ctx* ctx, int64_t rows, int width, const float* x, const float* w, const float* b, float* y);
+/* test hooks: the kernels on fp16 parts that the tower runs on where its weights allow.  A value v
+ * times a power of two s (at most 2^15 in all) is hi = fp16(s v), lo = fp16(s v - hi); a split row
+ * of KP values (a multiple of 64) is, for every 32 of them, their 32 hi and then their 32 lo halves.
+ * exn_vis_gemm_s: Y (M x N) = DESCALE X W^T + BIAS (+ R), X M split rows, W fp16 in KP / 32 runs of
+ * N rounded up to 64 rows of 32; or, YS given, through GELU (ACT as exn_vis_gemm), times OSCALE,
+ * into split rows of LDY; or, PARTS over 1, DESCALE X W^T alone as the PARTS sums of K's shares, M N
+ * floats each after the last.  exn_vis_gemm_way (needs no GPU): which TILE that runs on (0 .. 6), and
+ * how many parts pay.  exn_vis_ln_s: X (ROWS x WIDTH) += BIAS + the PARTS sums (PARTS 0: none), then
+ * LayerNorm, times SCALE as split rows YS or as it is into YF.  exn_vis_heads_s: QKV rows (N x
+ * 3 HEADS 72) with the rotary CS (N x 144: 72 cosines, 72 sines), times QS, KS, VS, into split heads:
+ * Q, K [head][N] of 152 halves (72 hi, 72 lo, 8 unused), VT two planes (hi, lo) of [head][72][N
+ * rounded up to 64].  exn_vis_attend_s: attention on them, SC taking the scores' scale off (they come
+ * in log2 units), into split rows YS of 72 HEADS at VT's scale, or times VDE into YF.
+ * exn_vis_spread: for LayerNorm gains G and shifts B (PERIOD of them, repeated along W's COLS), A2 =
+ * G^2 + B^2, T2 (ROWS) the mean squares of W x + BIAS (or of its GELU), SPREAD2 (2 doubles) [0] the
+ * largest |w_j|^2 over the mean square of w_j x.  Doubles. */
+int exn_vis_gemm_way(int64_t m, int64_t n, int64_t kp, int parts, int* tile, int* pays);
+int exn_vis_gemm_s(exn_ctx* ctx, const uint16_t* x, const uint16_t* w, const float* bias, const float* r, float* y,
+                   uint16_t* ys, int64_t m, int64_t n, int64_t kp, float descale, float oscale, int64_t ldy, int act,
+                   int parts);
+int exn_vis_ln_s(exn_ctx* ctx, int64_t rows, int width, float* x, int parts, const float* part, const float* bias,
+                 const float* w, const float* b, float scale, uint16_t* ys, float* yf);
+int exn_vis_heads_s(exn_ctx* ctx, int n, int heads, const float* qkv, const float* cs, float qs, float ks, float vs,
+                    uint16_t* q, uint16_t* k, uint16_t* vt);
+int exn_vis_attend_s(exn_ctx* ctx, int n, int heads, const uint16_t* q, const uint16_t* k, const uint16_t* vt, float sc,
+                     float vde, uint16_t* ys, float* yf);
+int exn_vis_spread(exn_ctx* ctx, int rows, int cols, const float* w, const float* g, const float* b, int period,
+                   const float* bias, int gelu, double* a2, double* t2, double* spread2);
 
 /* --- the prompt encoder (replaces illatio's qwen3 forward under src/encoder.lisp:41-67,143-183) ---
  * Qwen3-VL-8B's text model read for every token's state after its last block, before the final

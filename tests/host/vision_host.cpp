@@ -54,7 +54,6 @@ hipError_t round_f16(hipStream_t, int64_t, float*) { return hipSuccess; }
 hipError_t synth_normal(hipStream_t, uint64_t, int64_t, float, float, int, float*) { return hipSuccess; }
 hipError_t vis_sum(hipStream_t, int64_t, const float*, const float*, float*) { return hipSuccess; }
 hipError_t vis_prep(hipStream_t, const float*, int, int, int, const float*, int, int, float*, float*, float*) { return hipSuccess; }
-hipError_t vis_ln(hipStream_t, int64_t, int, const float*, const float*, const float*, float*) { return hipSuccess; }
 hipError_t vis_ln_s(hipStream_t, int64_t, int, int, float*, int, const float*, const float*, const float*, const float*, float,
                     uint16_t* ys, float*) {
   return note(ys ? "ln/s" : "ln/f");
@@ -67,6 +66,7 @@ hipError_t vis_gemm_s(hipStream_t, const uint16_t*, const uint16_t*, const float
   return note("mm/s");
 }
 int vis_split(int64_t, int64_t, int64_t) { return 2; }
+int vis_tile(int64_t, int64_t, int64_t, int) { return 0; }
 hipError_t vis_gemm_part(hipStream_t, const uint16_t*, const uint16_t*, float*, int64_t, int64_t, int64_t, float, int) {
   return note("mm/s");
 }

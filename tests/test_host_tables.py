@@ -108,3 +108,26 @@ def test_convolutions_take_the_tiles_of_the_fewer_steps():
     assert conv_way(0, 64, 64, 1152, 1152, 1 << 26) == (1, 4, 256)
     assert conv_way(0, 1024, 1024, 144, 144, 0) == (1, 1, 4096)
     assert conv_way(0, 17, 4, 1152, 1152, 1 << 26) == (0, 4, 16)
+
+
+# --- the vision tower's split products: tiles ------------------------------------------------
+
+def gemm_way(m, n, kp, parts):
+    a, b = ctypes.c_int(), ctypes.c_int()
+    X.call("exn_vis_gemm_way", m, n, kp, parts, ctypes.byref(a), ctypes.byref(b))
+    return a.value, b.value
+
+
+def test_vision_split_cases_cover_the_tower():
+    """Every (kind, tile) of the tower's products at any patch count is among the cases that
+    test_gpu_vision_split.py runs, and those run on the tile they name."""
+    from vision_split_cases import CASES, padded
+    for kind, tile, m, n, parts in CASES:
+        assert gemm_way(m, n, padded(parts), parts)[0] == tile, (kind, tile, m, n, parts)
+    used = set()
+    for p in range(4, 16385, 4):
+        for kind, m, n, kp in (("f32", p, 3456, 1152), ("tanh", p, 4304, 1152), ("part", p, 1152, 1152),
+                               ("part", p, 1152, 4352), ("erf", p // 4, 4608, 4608), ("f32", p // 4, 4096, 4608)):
+            parts = gemm_way(m, n, kp, 1)[1] if kind == "part" else 1
+            used.add(("f32" if parts == 1 and kind == "part" else kind, gemm_way(m, n, kp, parts)[0]))
+    assert used <= {c[:2] for c in CASES}
