@@ -303,8 +303,8 @@ struct VaeEpi {
   // head's normed input; VAE_RMS writes yr only
   const float* gamma;
   uint16_t* yr;
-  // 1: k_conv's 256-pixel tiles always (its 128-pixel ones of large pictures off; the same sums, a test's
-  // switch)
+  // 1: k_conv's 256-pixel tiles always (its 128-pixel ones of large pictures off; the same sums, a
+  // test's switch)
   int wide_only;
 };
 // the tiles (SQUARE: k_conv_halo's), K split and workgroups of a 3 x 3 convolution with PARTS floats of

@@ -623,17 +623,18 @@ static hipError_t launch_halo(hipStream_t s, const uint16_t* x, const uint16_t* 
   return hipGetLastError();
 }
 
-// 128-pixel tiles of 4 waves (two workgroups a CU) for the 96- and 144-wide convolutions of
-// pictures of 2^18 pixels or more, where the output, residual and normed copy move as many bytes
-// as the products take time; 256-pixel tiles otherwise
+// k_conv on 128-pixel tiles of 4 waves (two workgroups a CU) for the 96- and 144-wide 1 x 1 and
+// stride-2 convolutions of pictures of 2^18 pixels or more, where the output, residual and normed copy
+// move as many bytes as the products take time; 256-pixel tiles otherwise (the 3 x 3 ones of such
+// pictures, whose sides are multiples of 16, are all k_conv_halo's)
 template <int BN, int TAPS, int UP, int OUT, int GAM = 0>
 static hipError_t launch_conv(hipStream_t s, const uint16_t* x, const uint16_t* wt, const float* bias, const VaeEpi& ep,
                               void* y, int h, int w, int c, int cout, int kp, ConvWay way = {false, 1}) {
   const int split = way.split;
   if constexpr (TAPS == 9 && UP < 2 && BN > 16)
     if (way.halo) return launch_halo<BN, UP, OUT, GAM>(s, x, wt, bias, ep, y, h, w, c, cout, kp, split);
-  if constexpr (BN == 96 || BN == 144) {
-    if (split == 1 && !ep.wide_only && (int64_t)h * w >= (1 << 18))
+  if constexpr ((BN == 96 || BN == 144) && (TAPS == 1 || UP == 2)) {
+    if (!ep.wide_only && (int64_t)h * w >= (1 << 18))
       return launch_conv1<BN, TAPS, UP, OUT, GAM, 4>(s, x, wt, bias, ep, y, h, w, c, cout, kp, 1);
   }
   return launch_conv1<BN, TAPS, UP, OUT, GAM, 8>(s, x, wt, bias, ep, y, h, w, c, cout, kp, split);

@@ -73,7 +73,7 @@ CONV_CASES = [  # (h, w, c, cout, taps, up, out, with res)
     (13, 7, 96, 192, 1, 0, 0, True),
     (21, 19, 64, 96, 1, 0, 0, False),   # encoder.conv1: a 1 x 1 product over RGBA neighbourhoods
     (6, 6, 768, 128, 9, 0, 1, False),   # the encoder's head: 128 of a 144-wide tile
-    # 2^18 pixels: the 128-pixel tiles of 4 waves, two workgroups a CU
+    # 2^18 pixels: two workgroups of 4 waves a CU, the 3 x 3 on 16 x 16 tiles, the 1 x 1 on 128 pixels
     (512, 512, 144, 144, 9, 0, 0, True),
     (512, 512, 96, 96, 9, 0, 1, False),
     (512, 512, 64, 96, 1, 0, 0, False),
@@ -376,18 +376,20 @@ def test_encode_rejects(ctx, enc_vae):
 
 
 def test_large_pictures_tiles_agree(ctx, enc_vae):
-    """Pictures of 2^18 pixels or more run their 96- and 144-wide convolutions on 128-pixel tiles
-    (the norm in the store, the residual, the first convolution's 1 x 1 included): a 32 x 32
-    latent's decode and a 512 x 512 picture's encode equal, bit for bit, the same on 256-pixel
-    tiles only."""
+    """Pictures of 2^18 pixels or more run their 96- and 144-wide 1 x 1 and stride-2 convolutions on
+    128-pixel tiles: a 32 x 32 latent's decode (the last stage's shortcut, 288 to 144) and a
+    1024 x 1024 picture's encode (the first convolution with the norm in its store; the first
+    stride 2, whose output has 2^18 pixels) equal, bit for bit, the same on 256-pixel tiles only.
+    The 3 x 3 convolutions run alike in both; test_conv_of_whole_neighbourhoods and the whole decodes
+    and encodes hold those to the oracle."""
     z = vo.synth_latent(33, 32, 32)
-    px = vo.synth_picture(34, 512, 512)
+    px = vo.synth_picture(34, 1024, 1024)
     a, _, _ = X.vae_decode(enc_vae, z, 32, 32)
-    la = X.vae_encode(enc_vae, px, 512, 512)
+    la = X.vae_encode(enc_vae, px, 1024, 1024)
     X.call("exn_vae_tiles", enc_vae.h, 0)
     try:
         b, _, _ = X.vae_decode(enc_vae, z, 32, 32)
-        lb = X.vae_encode(enc_vae, px, 512, 512)
+        lb = X.vae_encode(enc_vae, px, 1024, 1024)
     finally:
         X.call("exn_vae_tiles", enc_vae.h, 1)
     assert np.isfinite(a).all() and np.isfinite(la).all()
