@@ -768,8 +768,8 @@ static int velocity(exn_dit* d, const float* context, int ptext, const float* la
   int8_t* xq = nullptr;
   uint16_t* xd = nullptr;
   if (d->int8) {
-    TRY(dit_buf(d, "i8q", (size_t)(std::max<int64_t>(l, 256) * EXN_F), (void**)&xq));
-    TRY(dit_buf(d, "i8d", (size_t)(std::max<int64_t>(l, 256) * (EXN_F / 32)) * 2, (void**)&xd));
+    TRY(dit_buf(d, "i8q", (size_t)(std::max<int64_t>(l, 256) * EXN_W), (void**)&xq));
+    TRY(dit_buf(d, "i8d", (size_t)(std::max<int64_t>(l, 256) * (EXN_W / 32)) * 2, (void**)&xd));
   }
   // an edge product in fp32: Y (m rows, ldy apart) = X (m rows of the matrix's inputs) W^T
   auto edge_mm = [&](int e, const float* xin, int64_t m, float* yout, int gelu) {
