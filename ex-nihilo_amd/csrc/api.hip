@@ -265,9 +265,10 @@ static hipError_t rows_mm(hipStream_t s, const exn_w* w, const uint16_t* x, int6
 // them) apart -- with K split over the chip when they are about one row of tiles, else by
 // rows_mm (an edit's 4608 prompt rows through to_out and down: 288 tiles) -- and the image
 // rows after them by rows_mm, so that the 4096 image rows of a 1024^2 picture fill whole
-// waves.  The image rows are tiled alike in every pass whatever comes before them, and a tile's
-// rows are the same bits however the rows are tiled, so a cached pass's image rows match the
-// uncached pass's.
+// waves.  The image rows are tiled alike in every pass whatever comes before them, so a cached
+// pass's image rows match the uncached pass's bit for bit.  (More than 48 rows are the same bits
+// however they are tiled; at most 48 are summed by four waves, every fourth k-step each, and so in
+// another order than the same rows among more.)
 hipError_t block_mm(hipStream_t s, const exn_w* w, const uint16_t* x, int64_t lda, int64_t n, int64_t nh,
                            Epi epi, const EpiArgs& ea, float* part) {
   if (nh > 0 && nh < n) {

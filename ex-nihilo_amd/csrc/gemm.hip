@@ -1667,7 +1667,8 @@ hipError_t gemm_split_rows(hipStream_t s, const uint16_t* x, int64_t lda, const 
   if (!epi_ok) return hipErrorNotSupported;
   if (few_fits(x, lda, w, M, N, K, ea) && a16(part)) {
     // at most 256 rows: the few-row tiles, K split so that the tiles' workgroups are about one a
-    // CU, each at least 4 k-steps, at most SMAX ways and within PART_CAP
+    // CU (at most 48 rows: rows_split's count), each at least 4 k-steps, at most SMAX ways and within
+    // PART_CAP
     const int64_t tiles = N / (M > 128 ? 128 : 256);
     int64_t S = M <= ROWS_MAX ? rows_split(M, N, K, smax) : 256 / tiles;
     if (S > K / 256) S = K / 256;

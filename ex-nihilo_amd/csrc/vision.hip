@@ -13,8 +13,8 @@
 // fp32 MFMAs (157 TFLOP/s dense on MI355X) keep the reference's fp32 products: the tower is
 // held to float32 numpy, not to a bf16 tolerance.  Where the weights are fp16 or bf16 values, as
 // every mmproj file's are, the blocks run on vision_split.hip's kernels, faster and nearer to the
-// exact values; those here take the patch embedding, whose input has no bound, and the products of
-// weights that fp16 does not hold.
+// exact values; those here take the patch embedding, whose input has no bound, and the products and
+// heads of weights that fp16 does not hold or whose bounds are far above most inputs.
 #include "exn_common.h"
 
 namespace exn {

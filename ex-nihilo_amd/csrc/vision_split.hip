@@ -3,14 +3,18 @@
 // lo = fp16(s X - hi), with s a power of two that keeps |s X| at or below 2^15.  hi + lo carries
 // 23 to 24 significant bits of every value down to 2^-16 of the bound s was made for, and an
 // absolute error of 2^-40 of the bound below that, so a product over the two parts rounds like
-// the fp32 one (the sums stay in fp32 inside the MFMA).  The weights of an mmproj-f16 file are
-// fp16 values, and bf16 ones become fp16 values times a power of two: exact in one part, so
+// the fp32 one (the sums stay in fp32 inside the MFMA) as long as the bound is not far above what
+// most values have, which the weights tell (k_vis_rows; api_vision.hip's kVisSpread): where it is, the
+// product runs in fp32.  The weights of an mmproj-f16 file are fp16 values, and bf16 ones are fp16
+// values times a power of two where a matrix's smallest are within about 2^-31 of its largest (one
+// below leaves the product in fp32): exact in one part, so
 // Y = X W^T takes two fp16 MFMAs (hi, lo) where v_mfma_f32_16x16x4_f32 needed eight of twice the
 // length: 16 times the rate over 2.  The bounds come from the weights alone (api_vision.hip):
 // LayerNorm's output is at most sqrt(D) max|g| + max|b| whatever its input.
 //
 //   k_vis_stats   max |x| and the largest row norm of a tensor, for the bounds;
 //   k_vis_pack    a matrix as fp16 rows, a flag when a value is not exact;
+//   k_vis_square, k_vis_rows  the sizes that inputs and outputs have, from the weights;
 //   k_vis_gemm_s  Y = X W^T + b (+ R) (then GELU), X split, W fp16;
 //   k_vis_ln_s    LayerNorm into split rows, over the sum of a split product's parts;
 //   k_vis_heads_s QKV rows into split heads, the rotary applied;
