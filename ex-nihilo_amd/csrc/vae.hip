@@ -370,8 +370,8 @@ k_conv(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Wt, const fl
 // chunk, of the next chunk's neighbourhood goes out.  Channels past C read as zeros.
 // Measured (us, k_conv then this): 288 -> 288 at 512 x 512 508 / 458, 576 -> 576 at 256 x 256 429 /
 // 371, 144 -> 144 at 1024 x 1024 733 / 662 with its fp32 output and 689 / 514 without, upsampling
-// 288 at 1024 x 1024 2011 / 1751, 96 -> 96 at 1024 x 1024 370 / 268; decode 19.6 -> 17.2 ms, encode
-// 5.5 -> 4.8.  What is left runs at about 1.05 PFLOP/s, the chip's power at this mix of reads.
+// 288 at 1024 x 1024 2011 / 1751, 96 -> 96 at 1024 x 1024 370 / 268; decode 19.6 -> 17.4 ms, encode
+// 5.5 -> 4.9.  What is left runs at about 1.05 PFLOP/s, the chip's power at this mix of reads.
 template <int BN>
 struct HaloTile {
   static constexpr int WNC = BN % 144 == 0 ? 144 : 96, NJ = WNC / 16, NWN = BN / WNC, NWM = 4, NW = NWM * NWN, MI = 4;
