@@ -280,7 +280,7 @@ k_vis_ln_s(int width, int kp, float* __restrict__ x, int S, int64_t mn, const fl
 hipError_t vis_ln_s(hipStream_t s, int64_t rows, int width, int kp, float* x, int S, const float* part,
                     const float* bias, const float* w, const float* b, float scale, uint16_t* ys, float* yf) {
   if (rows <= 0) return hipSuccess;
-  if (width <= 0 || width % 4 || width > 5120 || S < 0 || !ys == !yf) return hipErrorInvalidValue;
+  if (width % 4 || width > 5120 || S < 0 || !ys == !yf) return hipErrorInvalidValue;
   if (ys && (width % 64 || kp != width)) return hipErrorInvalidValue;   // no columns past the width to clear
   hipLaunchKernelGGL(k_vis_ln_s, dim3((unsigned)rows), dim3(256), 0, s, width, kp, x, S, rows * width, part, bias, w, b,
                      scale, ys, yf);
